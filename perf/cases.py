@@ -267,7 +267,7 @@ def tolerance(case):
     # bf16 activations between the projections (and bf16 weights on the matrix
     # cores): 0.0018 to 0.0019 from the results in 64 bits with the residual
     # added, 0.0034 to 0.0059 without.
-    return {"rel": 8e-3 if case["norm"] else 2e-2}
+    return {"rel": 8e-3 if case["norm"] else 1e-2}
 
 
 # ----------------------------------------------------- the results in 64 bits

@@ -491,6 +491,12 @@ int switch_call(const rmoe_qweight* gate_up, const rmoe_qweight* down, const uin
     a.score_stride = top_k;
     a.residual = residual;
   }
+  // the few-token kernels at their shape (3 tokens x 8 slots, 4 bits:
+  // gate/up and down 10.0 + 6.4 us against 10.8 + 13.8 of the general ones)
+  if (tokens <= rmoe::kFewMaxTokens && tokens * top_k < rmoe::kPrefillMinRows &&
+      top_k <= rmoe::kMaxFusedRouted && H == rmoe::kFusedH && I == rmoe::kFusedI &&
+      aligned(gate_up->scales, 4) && aligned(gate_up->biases, 4))
+    a.few_bits = gate_up->bits;
   hipError_t e = rmoe::launch_gate_up(a, gate_up->bits, s);
   if (e != hipSuccess) return hip_fail(e, "gate/up launch");
   e = rmoe::launch_down(a, gate_up->bits, combine, s);

@@ -1370,7 +1370,7 @@ __global__ __launch_bounds__(256) void gate_up_few_kernel(const DecodeArgs p) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   // the router launch before this one has finished with the call's tag
-  if (blockIdx.x == 0 && threadIdx.x == 0)
+  if (!p.switch_mode && blockIdx.x == 0 && threadIdx.x == 0)
     store_coherent_u32(&p.fs->epoch, load_coherent_u32(&p.fs->epoch) + 1);
   const int gw = blockIdx.x * 4 + wave;
   const int m = gw / few::kWavesPerUnit;

@@ -126,3 +126,38 @@ def test_few_token_graph_replays_equal_eager_calls(torch_cuda, bits):
         torch.cuda.synchronize()
         assert torch.equal(eager, ref_a)
     assert native.workspace_status(ws) == 0
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("T,k", [(1, 8), (2, 1), (3, 8), (5, 7), (7, 8), (8, 7)])
+def test_few_token_switch(torch_cuda, bits, T, k):
+    """A caller's routing at the few-token shape: repeated experts, ids
+    outside the bank, per-slot rows and the weighted combine with a residual.
+    Same bounds as the block above."""
+    torch = torch_cuda
+    from helpers import bank_to_dev, dev_i32
+    from runnel_amd import native
+    print(f"few-token switch bits={bits} T={T} k={k}", flush=True)
+    L = M.make_layer(900 + T + bits, hidden=2048, inter=512, experts=12, top_k=k, bits=bits,
+                     shared=False)
+    x = M.make_x(40 + T, T, 2048)
+    idx = np.random.default_rng(T * k).integers(0, 12, (T, k)).astype(np.int32)
+    bad = np.zeros_like(idx, bool)
+    bad[T - 1, k - 1] = T > 1
+    given = np.where(bad, np.int32(12), idx)
+    given[bad & (idx % 2 == 1)] = -1
+    keep = (bank_to_dev(L.gate_up), bank_to_dev(L.down))
+    gu, dn = (native.qweight_struct(*b, bits) for b in keep)
+    y = native.switch_glu(dev_bf16(x), dev_i32(given), gu, dn)
+    ref, mlx = (M.switch_glu(L, x, idx, mode=m) for m in ("contract", "mlx"))
+    ref[bad] = mlx[bad] = 0.0
+    _check(host_bf16(y), M.f32_to_bf16(ref), M.f32_to_bf16(mlx))
+    assert not host_bf16(y)[bad].any()
+    w = np.random.default_rng(5).random((T, k)).astype(np.float32)
+    res = M.make_x(41 + T, T, 2048)
+    out = native.switch_combine(dev_bf16(x), dev_i32(given), torch.from_numpy(w).cuda(), gu, dn,
+                                residual=dev_bf16(res))
+    rows = M.bf16_to_f32(host_bf16(y)).astype(np.float64)
+    exp = M.round_bf16((rows * w[..., None]).sum(1).astype(np.float32))
+    exp = M.f32_to_bf16(M.bf16_to_f32(res) + exp)
+    _check(host_bf16(out), exp, exp)

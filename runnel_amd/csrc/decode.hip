@@ -1623,6 +1623,290 @@ __global__ __launch_bounds__(256) void qmv_kernel(const QmvArgs p,
   }
 }
 
+// ---------------------------------------------------------------- qmv rows
+// The same product for calls of many rows.  qmv_kernel reads an expert once
+// per row and is bound by its vector work, about six instructions per weight
+// and row (unpacking x, converting the codes, the multiply-adds); here up to
+// 16 rows of one expert share its weights on the matrix cores.
+//
+// The codes are converted to bf16, which holds them exactly, and multiplied
+// with x as they are.  Per 64-group, with c the middle code (8 or 128):
+//   acc += s (sum q x - c sum x) + (b + c s) sum x        in fp32,
+// the sum of x from an MFMA against ones and the first bracket from MFMAs
+// that start from -c sum x.  Nothing is rounded to 16 bits, and the middle
+// code keeps the two terms from cancelling: the error against 64 bits is
+// 0.75 to 0.98 of qmv_kernel's (K 256 to 4096, 8 and 4 bits).
+//
+// Workgroup: one group of up to 16 rows x CG NB 16 weight rows.  The rows
+// are those of one expert within a window of kQmvWindow rows, taken 16 at a
+// time; the workgroup of the first computes them, the others leave after one
+// round trip (DENSE: one matrix and rows in order, group j is rows 16 j ..
+// 16 j + 15).  A wave holds the rows' x for its slice of 256 values in
+// registers and walks NB blocks of 16 weight rows; the KS slices of a row
+// meet in LDS and are added pairwise.  A row's value depends on its own x
+// only, not on the rows it is grouped with.
+constexpr int kQmvWindow = 512;
+
+template <int BITS, int NB_>
+struct QmvRows {
+  static constexpr int L = 256;                    // values per slice
+  static constexpr int LV = BITS == 8 ? 64 : 128;  // values per weight load
+  static constexpr int NL = L / LV;                // weight loads per block
+  static constexpr int NF = L / 32;                // MFMA fragments per block
+  static constexpr int NG = L / 64;                // groups per block
+  static constexpr int NB = NB_;                   // blocks per wave
+  static constexpr int D = NB < 8 / NL ? NB : 8 / NL;  // blocks in flight
+  static constexpr int NGW = NG / 2;               // words of a block's scales
+};
+
+template <int BITS, int NB, bool DENSE>
+__global__ __launch_bounds__(1024) void qmv_rows_kernel(const QmvArgs p,
+                                                        const int blocks_per_row,
+                                                        const int KS) {
+  using S = QmvRows<BITS, NB>;
+  constexpr int L = S::L;
+  __shared__ int s_mem[16][16], s_x[16][16];
+  extern __shared__ f32x4_r s_part[];  // [waves][2][64] when KS > 1
+  const int group = blockIdx.x / blocks_per_row;
+  const int blk = blockIdx.x - group * blocks_per_row;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int col = lane & 15;
+  const int kg = lane >> 4;
+
+  const int n_wave = (blk * ((int)(blockDim.x >> 6) / KS) + wave / KS) * (16 * S::NB);
+  int e_m = -1, cnt;
+  if constexpr (DENSE) {
+    e_m = 0;
+    cnt = min(16, p.M - 16 * group);
+    if (lane < 16) s_mem[wave][lane] = s_x[wave][lane] = 16 * group + min(lane, cnt - 1);
+  } else {
+    const int m = group;
+    // ---- the rows of row m's expert in its window, in one round trip
+    struct Key {
+      int e, x;
+    };
+    auto key_of = [&](int i) {
+      const int x = p.lhs ? p.lhs[i] : i;
+      const int e = p.rhs ? p.rhs[i] : 0;
+      // out of range: a row of zeros that shares nothing
+      const bool ok = (unsigned)x < (unsigned)p.x_rows && (unsigned)e < (unsigned)p.experts;
+      return Key{ok ? e : -1, ok ? x : 0};
+    };
+    const int w0 = m & ~(kQmvWindow - 1);
+    const int w1 = min(p.M, w0 + kQmvWindow);
+    Key keys[kQmvWindow / 64];
+#pragma unroll
+    for (int j = 0; j < kQmvWindow / 64; ++j)
+      if (w0 + 64 * j < w1) keys[j] = key_of(min(w0 + 64 * j + lane, w1 - 1));
+#pragma unroll
+    for (int j = 0; j < kQmvWindow / 64; ++j)
+      if ((m - w0) >> 6 == j) e_m = __builtin_amdgcn_readlane(keys[j].e, m & 63);
+    if (e_m < 0) {
+      // zeros, each wave its own columns
+      for (int n = n_wave + lane; n < min(n_wave + 16 * S::NB, p.N); n += 64) {
+        if (p.y_f32)
+          p.y_f32[(size_t)m * p.N + n] = 0.0f;
+        else
+          p.y_bf16[(size_t)m * p.N + n] = 0;
+      }
+      return;
+    }
+    int rank_m = 0, seen = 0;
+#pragma unroll
+    for (int j = 0; j < kQmvWindow / 64; ++j) {
+      const int i0 = w0 + 64 * j;
+      if (i0 < w1) {
+        const uint64_t same = __ballot(keys[j].e == e_m && i0 + lane < w1);
+        if ((m - w0) >> 6 == j)
+          rank_m = seen + __popcll(same & ((1ull << (m & 63)) - 1ull));
+        seen += __popcll(same);
+      }
+    }
+    if (rank_m & 15) return;  // an earlier row's workgroup computes row m
+    cnt = min(16, seen - rank_m);
+    seen = 0;
+#pragma unroll
+    for (int j = 0; j < kQmvWindow / 64; ++j) {
+      const int i0 = w0 + 64 * j;
+      if (i0 < w1) {
+        const bool mine = keys[j].e == e_m && i0 + lane < w1;
+        const uint64_t same = __ballot(mine);
+        const int at = seen + __popcll(same & ((1ull << lane) - 1ull)) - rank_m;
+        if (mine && at >= 0 && at < 16) {
+          s_mem[wave][at] = i0 + lane;
+          s_x[wave][at] = keys[j].x;
+        }
+        seen += __popcll(same);
+      }
+    }
+  }
+
+  // ---- weights: block b of the wave is rows n_wave + 16 b + col
+  const int ks = wave % KS;
+  const int K = p.K;
+  const size_t bank = (size_t)e_m * p.N;
+  const int WPR = K * BITS / 32;
+  const int G = K >> 6;
+  uint4 ring[S::D][S::NL];
+  uint32_t sr[S::D][S::NGW], br[S::D][S::NGW];
+  auto load_params = [&](int b, uint32_t (&s)[S::NGW], uint32_t (&bb)[S::NGW]) {
+    const size_t row = bank + min(n_wave + 16 * b + col, p.N - 1);
+    const size_t o = row * G + ks * S::NG;
+    __builtin_memcpy(s, __builtin_assume_aligned(p.w.s + o, 2 * S::NG), 2 * S::NG);
+    __builtin_memcpy(bb, __builtin_assume_aligned(p.w.b + o, 2 * S::NG), 2 * S::NG);
+  };
+  auto load_w = [&](int b, int c) {
+    const size_t row = bank + min(n_wave + 16 * b + col, p.N - 1);
+    return load16(p.w.w + row * WPR + (ks * S::NL + c) * 16 + kg * 4);
+  };
+#pragma unroll
+  for (int d = 0; d < S::D; ++d) {
+    load_params(d, sr[d], br[d]);
+#pragma unroll
+    for (int c = 0; c < S::NL; ++c) ring[d][c] = load_w(d, c);
+  }
+
+  // ---- x fragments: lane (row col, kg); 4-bit codes leave a word as 0, 2, 4,
+  // 6, 1, 3, 5, 7 and a group's four lane quarters hold 16 of its values
+  // each, so x takes the same order
+  const int xr = s_x[wave][col < cnt ? col : 0];
+  const uint16_t* x0 = p.x + (size_t)xr * K + ks * L;
+  bf16x8_r a[S::NF];
+#pragma unroll
+  for (int f = 0; f < S::NF; ++f) {
+    const int k = BITS == 8 ? 64 * (f >> 1) + 16 * kg + 8 * (f & 1)
+                            : 64 * (f >> 1) + 32 * (kg & 1) + 16 * (kg >> 1) + 8 * (f & 1);
+    const uint4 v = load16(x0 + k);
+    u32x4 o;
+    if constexpr (BITS == 8) {
+      o = u32x4{v.x, v.y, v.z, v.w};
+    } else {
+      o.x = __builtin_amdgcn_perm(v.y, v.x, 0x05040100u);
+      o.y = __builtin_amdgcn_perm(v.w, v.z, 0x05040100u);
+      o.z = __builtin_amdgcn_perm(v.y, v.x, 0x07060302u);
+      o.w = __builtin_amdgcn_perm(v.w, v.z, 0x07060302u);
+    }
+    a[f] = __builtin_bit_cast(bf16x8_r, o);
+  }
+  auto mfma = [](const bf16x8_r& aa, const bf16x8_r& bb, const f32x4_r& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(aa, bb, c, 0, 0, 0);
+  };
+  // -c sum x of every group, as the accumulators hold it (rows 4 kg + i)
+  constexpr float kMid = BITS == 8 ? 128.0f : 8.0f;
+  const bf16x8_r ones = __builtin_bit_cast(
+      bf16x8_r, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+  f32x4_r cx[S::NG];
+#pragma unroll
+  for (int g = 0; g < S::NG; ++g) {
+    cx[g] = mfma(a[2 * g], ones, f32x4_r{0.f, 0.f, 0.f, 0.f});
+    cx[g] = mfma(a[2 * g + 1], ones, cx[g]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cx[g][i] *= -kMid;
+  }
+
+  f32x4_r acc[S::NB];
+#pragma unroll
+  for (int b = 0; b < S::NB; ++b) {
+    acc[b] = f32x4_r{0.f, 0.f, 0.f, 0.f};
+    f32x4_r even;
+    const int d = b % S::D;
+#pragma unroll
+    for (int c = 0; c < S::NL; ++c) {
+      const uint4 w = ring[d][c];
+      constexpr int GL = S::LV / 64;  // groups per load
+      bf16x8_r bf[2 * GL];
+      if constexpr (BITS == 8) {
+        const u32x4 lo = {codes_bf16x2(w.x, 0), codes_bf16x2(w.x, 1), codes_bf16x2(w.y, 0),
+                          codes_bf16x2(w.y, 1)};
+        const u32x4 hi = {codes_bf16x2(w.z, 0), codes_bf16x2(w.z, 1), codes_bf16x2(w.w, 0),
+                          codes_bf16x2(w.w, 1)};
+        bf[0] = __builtin_bit_cast(bf16x8_r, lo);
+        bf[1] = __builtin_bit_cast(bf16x8_r, hi);
+      } else {
+        // lanes 32-63 hold the second group's codes: swap halves so that a
+        // fragment is one group
+        const auto e = __builtin_amdgcn_permlane32_swap(w.x, w.z, false, false);
+        const auto o = __builtin_amdgcn_permlane32_swap(w.y, w.w, false, false);
+        const uint32_t q[4] = {(uint32_t)e[0], (uint32_t)o[0], (uint32_t)e[1], (uint32_t)o[1]};
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+          const uint32_t lo = q[f] & 0x0F0F0F0Fu, hi = (q[f] >> 4) & 0x0F0F0F0Fu;
+          auto pk = [](uint32_t v, bool up) {
+            // a byte 0..15 is e4m3 q 2^-9, scaled back exactly
+            const bf16x2_t r = up ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.0f, true)
+                                  : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.0f, false);
+            return __builtin_bit_cast(uint32_t, r);
+          };
+          const u32x4 v = {pk(lo, false), pk(lo, true), pk(hi, false), pk(hi, true)};
+          bf[f] = __builtin_bit_cast(bf16x8_r, v);
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < GL; ++g) {
+        const int gi = c * GL + g;
+        f32x4_r dq = mfma(a[2 * gi], bf[2 * g], cx[gi]);
+        dq = mfma(a[2 * gi + 1], bf[2 * g + 1], dq);
+        const float s = gi & 1 ? bf16_hi(sr[d][gi >> 1]) : bf16_lo(sr[d][gi >> 1]);
+        const float bi = gi & 1 ? bf16_hi(br[d][gi >> 1]) : bf16_lo(br[d][gi >> 1]);
+        const float bm = fmaf(bi, -1.0f / kMid, -s);  // -(b + c s) / c
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dq[i] = fmaf(s, dq[i], bm * cx[gi][i]);
+        // (pairs of groups first: fewer roundings at the sum's size)
+        if (gi % 2 == 0) even = dq;
+        else acc[b] += even + dq;
+      }
+      if (b + S::D < S::NB) ring[d][c] = load_w(b + S::D, c);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (b + S::D < S::NB) load_params(b + S::D, sr[d], br[d]);
+  }
+
+  // ---- the KS slices meet in LDS two blocks at a time and are added pairwise,
+  // block b by the wave of slice b % KS
+  const int cgw = (wave / KS) * KS;  // first wave of the column group
+#pragma unroll
+  for (int b = 0; b < S::NB; ++b) {
+    f32x4_r v = acc[b];
+    if (KS > 1) {
+      if (b % 2 == 0) {
+        if (b > 0) __syncthreads();
+        s_part[(wave * 2) * 64 + lane] = acc[b];
+        if (b + 1 < S::NB) s_part[(wave * 2 + 1) * 64 + lane] = acc[min(b + 1, S::NB - 1)];
+        __syncthreads();
+      }
+      if (b % KS != ks) continue;
+      const f32x4_r* sp = s_part + (cgw * 2 + b % 2) * 64 + lane;
+      // pairwise: fours, then the fours
+      f32x4_r four[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        four[q] = f32x4_r{0.f, 0.f, 0.f, 0.f};
+        if (4 * q < KS) {
+          f32x4_r t[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            t[j] = 4 * q + j < KS ? sp[(4 * q + j) * 2 * 64] : f32x4_r{0.f, 0.f, 0.f, 0.f};
+          four[q] = (t[0] + t[1]) + (t[2] + t[3]);
+        }
+      }
+      v = (four[0] + four[1]) + (four[2] + four[3]);
+    }
+    const int n = n_wave + 16 * b + col;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 4 * kg + i;
+      if (r < cnt && n < p.N) {
+        const size_t o = (size_t)s_mem[wave][r] * p.N + n;
+        if (p.y_f32)
+          p.y_f32[o] = v[i];
+        else
+          p.y_bf16[o] = (uint16_t)f32_to_bf16(v[i]);
+      }
+    }
+  }
+}
+
 // ------------------------------------------------------------------ launch
 #define RMOE_CHECK_LAUNCH()                  \
   do {                                       \
@@ -1833,7 +2117,44 @@ static hipError_t qmv_cpl(const QmvArgs& a, hipStream_t s) {
   return hipSuccess;
 }
 
+// When a call takes qmv_rows_kernel (its slices are 256 values, up to
+// sixteen, their group parameters words of 8 bytes), us against qmv_kernel,
+// experts of 512 x 2048 / 2048 x 512 / 512 x 4096 (N x K):
+//   gathered rows, 4 bits: 64 rows 16.9 -> 12.0, 16.8 -> 11.4, 25.4 -> 25.7;
+//     130: 29.6 -> 22.7, 28.7 -> 20.1, 44.2 -> 38.8; 320: 74.9 -> 45.2,
+//     71.9 -> 38.1, 124 -> 64
+//   8 bits: 96 rows 24.5 -> 25.8, 30.7 -> 21.7; 130: 29.9 -> 28.5, 38.5 ->
+//     24.4, 53.0 -> 49.6; 320: 84 -> 57, 103 -> 49, 148 -> 69
+//   small products lose (96 rows of 1024 x 256: 7.4 -> 7.8)
+//   one matrix, 40 rows: 10.9 -> 5.4, 10.4 -> 4.3, 16.2 -> 8.4; 16 rows of
+//     512 x 4096 at 8 bits lose (7.5 -> 9.0)
+static bool qmv_rows_ok(const QmvArgs& a, int bits) {
+  if (a.K % 256 || a.K > 4096 || (((uintptr_t)a.w.s | (uintptr_t)a.w.b) & 7)) return false;
+  if (!a.lhs && !a.rhs) return a.M >= 32;
+  const bool many = a.M >= 128 || (a.M >= 64 && a.K <= (bits == 4 ? 2048 : 1024));
+  return many && (long long)a.M * a.N * a.K >= 1ll << 25;
+}
+
+template <int BITS, int NB, bool DENSE>
+static hipError_t qmv_rows(const QmvArgs& a, hipStream_t s) {
+  const int ks = a.K / QmvRows<BITS, NB>::L;
+  const int cg = ks <= 4 ? 4 / ks : 1;
+  const int per = 16 * NB * cg;
+  const int bpr = (a.N + per - 1) / per;
+  const long long groups = DENSE ? (a.M + 15) / 16 : a.M;
+  const size_t lds = ks > 1 ? (size_t)ks * cg * 2 * 64 * sizeof(f32x4_r) : 0;
+  hipLaunchKernelGGL((qmv_rows_kernel<BITS, NB, DENSE>), dim3((unsigned)(bpr * groups)),
+                     dim3(64 * ks * cg), lds, s, a, bpr, ks);
+  RMOE_CHECK_LAUNCH();
+  return hipSuccess;
+}
+
 hipError_t launch_qmv(const QmvArgs& a, int bits, hipStream_t s) {
+  if (qmv_rows_ok(a, bits)) {
+    if (!a.lhs && !a.rhs)
+      return bits == 8 ? qmv_rows<8, 1, true>(a, s) : qmv_rows<4, 1, true>(a, s);
+    return bits == 8 ? qmv_rows<8, 4, false>(a, s) : qmv_rows<4, 4, false>(a, s);
+  }
   const int vpc = bits == 8 ? 16 : 32;
   const int cpl = (a.K / vpc + 63) / 64;
   if (bits == 8) {

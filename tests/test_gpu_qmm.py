@@ -94,3 +94,51 @@ def test_dense_qmm_random_shapes(torch_cuda, bits, shape):
     ref64, x, _, wb = _bf16_weight_product(xb, words, s, b, bits)
     nbad, _ = _check_contract(host_bf16(y), ref64, x, wb)
     assert nbad == 0
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("Mr,N,K,E", [
+    (32, 80, 256, 1), (40, 512, 2048, 1), (63, 130, 3072, 1),      # one matrix
+    (64, 2048, 512, 8), (130, 1100, 256, 3), (530, 144, 512, 40),  # gathered
+    (128, 520, 512, 1), (300, 64, 2048, 200), (128, 72, 4096, 5)])
+def test_rows_sharing_experts(torch_cuda, bits, Mr, N, K, E):
+    """Many rows a call, fp32 out: row groups that fill, exceed or just miss
+    16, windows of 512 rows, column remainders, ids out of range (zero rows)
+    and 1 to 16 slices of K.  Every product and sum is fp32, so each output is
+    within K roundings of |x| . (|q - c| s + |b + c s|) of the 64-bit value
+    (c the middle code), and in norm far closer."""
+    torch = torch_cuda
+    from runnel_amd import native
+    rng = np.random.default_rng(Mr + N + K + bits)
+    w = rng.standard_normal((E, N, K), dtype=np.float32) * np.float32(0.02)
+    words, s, b = M.quantize(w, bits)
+    X = max(1, Mr // 3) if E > 1 or Mr >= 64 else Mr
+    xb = M.make_x(9 + Mr, X, K)
+    dev = (dev_i32(words), dev_bf16(s), dev_bf16(b))
+    if E == 1 and Mr < 64:
+        lhs, rhs = np.arange(Mr), np.zeros(Mr, np.int64)
+        y = native.gather_qmm(dev_bf16(xb), *(t[0] for t in dev), bits, out_dtype=torch.float32)
+    else:
+        lhs, rhs = rng.integers(0, X, Mr), rng.integers(0, E, Mr)
+        lhs[5], rhs[Mr - 1], rhs[17] = -1, E, -3
+        y = native.gather_qmm(dev_bf16(xb), *dev, bits,
+                              rhs_indices=torch.from_numpy(rhs.astype(np.int32)).cuda(),
+                              lhs_indices=torch.from_numpy(lhs.astype(np.int32)).cuda(),
+                              out_dtype=torch.float32)
+    got = y.cpu().numpy().astype(np.float64)
+    ok = (lhs >= 0) & (rhs >= 0) & (rhs < E)
+    assert not got[~ok].any()
+    x = M.bf16_to_f32(xb).astype(np.float64)[lhs * ok]
+    w64 = M.dequantize(words, s, b, bits, dtype=np.float64)
+    s64 = np.repeat(M.bf16_to_f32(s).astype(np.float64), 64, -1)
+    b64 = np.repeat(M.bf16_to_f32(b).astype(np.float64), 64, -1)
+    c = 2 ** (bits - 1)
+    size = np.abs(w64 - b64 - c * s64) + np.abs(b64 + c * s64)
+    ref = np.zeros_like(got)
+    bound = np.zeros_like(got)
+    for e in np.unique(rhs[ok]):
+        r = np.nonzero(ok & (rhs == e))[0]
+        ref[r], bound[r] = x[r] @ w64[e].T, np.abs(x[r]) @ size[e].T
+    err = np.abs(got - ref)
+    assert (err <= K * 2.0 ** -24 * bound).all()
+    assert np.linalg.norm(err) <= 4 * 2.0 ** -24 * np.linalg.norm(ref)

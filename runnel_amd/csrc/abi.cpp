@@ -710,7 +710,8 @@ int block_launch(const rmoe_layer* L, const uint16_t* x, int32_t tokens,
   a.scores_out = scores_out;
   if (few_eligible(L, tokens, lay.rows != 0)) a.few_bits = L->gate_up.bits;
   a.logit_planes = lay.rows ? rmoe::router_logit_planes(tokens) : 1;
-  if (lay.rows && rmoe::router_mfma_eligible(L->experts, L->hidden))
+  if (lay.rows && tokens > rmoe::router_direct_tokens(router_quantized(L)) &&
+      rmoe::router_mfma_eligible(L->experts, L->hidden))
     e = rmoe::launch_router_mfma(
         a, reinterpret_cast<float*>(static_cast<char*>(ws) + lay.wnorm),
         lay.split ? reinterpret_cast<uint16_t*>(static_cast<char*>(ws) + lay.split) : nullptr,

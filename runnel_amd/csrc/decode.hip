@@ -1918,6 +1918,18 @@ bool router_mfma_eligible(int E, int H) {
   return E % 64 == 0 && E <= 256 && H % 512 == 0 && H <= 4096;
 }
 
+// Tokens up to which the exact router in one launch beats logits and
+// selection (two launches, five with an 8-bit gate: split, both planes):
+// whole block in us, matrix-core router against router_kernel, 4 bits, at
+// hidden 2048 | 1024 | 4096 (256 | 128 | 64 experts).
+//   8-bit gate: 16 tokens 88.8 -> 66.8 | 49.4 -> 37.5 | 92.5 -> 70.6;
+//     48: 131.2 -> 127.2 | 54.0 -> 44.2 | 103.1 -> 81.3; 96: 150.0 -> 148.8 |
+//     57.8 -> 52.0 | 117.7 -> 97.4; 192: 162.0 -> 178.3 | 61.6 -> 63.4 | ..
+//   bf16 gate: 16 tokens 79.3 -> 76.2 | 42.5 -> 36.8 | 76.3 -> 70.3;
+//     24: 96.1 -> 94.8 | 44.7 -> 40.5 | 83.7 -> 77.6; 32: 102.9 -> 110.4 |
+//     45.3 -> 42.0 | 85.5 -> 79.8; 64: 129.4 -> 138.8 | 45.9 -> 52.2 | ..
+int router_direct_tokens(bool rq8) { return rq8 ? 96 : 24; }
+
 // 64 x 64 tiles (two workgroups of four waves per CU) from 4096 tokens on,
 // 32 x 32 below, where 64-token tiles leave most CUs idle: at 512 tokens
 // 11.7 against 17.3 us, at 8192 tokens 21.2 against 32.2 (event-timed).

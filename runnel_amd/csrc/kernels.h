@@ -136,6 +136,7 @@ hipError_t launch_rmsnorm(const uint16_t* x, const uint16_t* w, int T, int H, fl
                           uint16_t* out, hipStream_t s);
 // Many-token router on the matrix cores with exact selection (prefill).
 bool router_mfma_eligible(int E, int H);
+int router_direct_tokens(bool rq8);  // up to this many tokens launch_router is faster
 int router_logit_planes(int T);
 // wnorm: [E] floats; split: [2, E, H] bf16 (quantized gates only)
 hipError_t launch_router_mfma(const DecodeArgs& a, float* wnorm, uint16_t* split,

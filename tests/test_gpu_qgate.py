@@ -249,3 +249,27 @@ def test_prefill_router_widest_rows(torch_cuda):
     ref_idx, ref_scores, _ = M.route(x, L.router_w, 4)
     assert np.array_equal(idx.cpu().numpy(), ref_idx)
     assert np.abs(scores.cpu().numpy() - ref_scores).max() <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("router_bits,T", [(None, 16), (None, 24), (None, 25), (8, 16), (8, 95),
+                                           (8, 96), (8, 97)])
+def test_sorted_block_router_choice(torch_cuda, router_bits, T):
+    """Either side of the token counts where the expert-sorted block changes
+    from the one-launch router to the matrix-core one: routing bit-exact,
+    scores within one bf16 step (their contract) on both."""
+    torch = torch_cuda
+    from runnel_amd import native
+    print(f"sorted block router: gate bits {router_bits}, {T} tokens", flush=True)
+    L = M.make_layer(350 + T, hidden=512, inter=128, experts=64, top_k=4,
+                     router_bits=router_bits)
+    x = M.make_x(21 + T, T, 512)
+    h = layer_to_dev(L)
+    for _ in range(2):  # the second call finds the first one's counters
+        out, idx, scores = native.moe_block(h, dev_bf16(x), return_routing=True)
+        torch.cuda.synchronize()
+        ref, ref_idx, ref_scores = M.block_forward(L, x, mode="prefill")
+        assert np.array_equal(idx.cpu().numpy(), ref_idx)
+        assert np.abs(scores.cpu().numpy() - ref_scores).max() <= 2.0 ** -8
+        got, r = M.bf16_to_f32(host_bf16(out)), M.bf16_to_f32(ref)
+        assert cosine(got.reshape(-1), r.reshape(-1)) >= MIN_COS
+        assert np.abs(got - r).max() <= MAX_ABS

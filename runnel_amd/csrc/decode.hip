@@ -622,33 +622,36 @@ typedef float f32x4_r __attribute__((ext_vector_type(4)));
 // buffer nobody reads), so NB - 2 stages' loads may stay in flight when a
 // stage's own copy is needed.
 //
-// ACC adds the sums already in `logits` (the second plane of a split gate).
+// PL planes of router rows (a split gate's two) share each stage's token rows
+// and accumulators: one pass per plane took 14 + 17 us at 1750 tokens, both
+// in one 17.
 // WNORM: the first token tile's workgroups also write the bound
 // ||w_e||_2 (1 + 2^-10) of their router rows into wnorm from the fragments
 // they read (the padding covers any order of the fp32 sum of squares).
 __device__ __forceinline__ int stage_swizzle(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
-template <int BT, int BE, int WM, int WN>
+template <int BT, int BE, int WM, int WN, int PL>
 struct LogitsTile {
-  static constexpr int WAVES = WM * WN, ROWS = BT + BE, NI = ROWS / 8, ND = NI / WAVES;
+  static constexpr int WAVES = WM * WN, ROWS = BT + PL * BE, NI = ROWS / 8, ND = NI / WAVES;
   static constexpr int MBW = BT / WM / 16, CBW = BE / WN / 16;
   static_assert(NI % WAVES == 0 && MBW >= 1 && CBW >= 1, "tile shape");
   static constexpr int vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 };
 
-template <int BT, int BE, int WM, int WN, bool WNORM>
+template <int BT, int BE, int WM, int WN, int PL, bool WNORM>
 __device__ __forceinline__ void logits_stage(
     const uint16_t* __restrict__ buf, const int (&rd)[2], int arow0, int brow0,
-    f32x4_r (&acc)[LogitsTile<BT, BE, WM, WN>::MBW][LogitsTile<BT, BE, WM, WN>::CBW],
-    float (&ss)[LogitsTile<BT, BE, WM, WN>::CBW], bool norms) {
-  using C = LogitsTile<BT, BE, WM, WN>;
+    f32x4_r (&acc)[LogitsTile<BT, BE, WM, WN, PL>::MBW][LogitsTile<BT, BE, WM, WN, PL>::CBW],
+    float (&ss)[LogitsTile<BT, BE, WM, WN, PL>::CBW], bool norms) {
+  using C = LogitsTile<BT, BE, WM, WN, PL>;
   const char* b = reinterpret_cast<const char*>(buf);
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    u32x4 bf[C::CBW];
+    u32x4 bf[PL * C::CBW];  // plane by plane
 #pragma unroll
-    for (int cb = 0; cb < C::CBW; ++cb)
-      bf[cb] = *reinterpret_cast<const u32x4*>(b + (brow0 + cb * 16) * 128 + rd[j]);
+    for (int cb = 0; cb < PL * C::CBW; ++cb)
+      bf[cb] = *reinterpret_cast<const u32x4*>(
+          b + (brow0 + (cb / C::CBW) * BE + (cb % C::CBW) * 16) * 128 + rd[j]);
     if (WNORM && norms) {
 #pragma unroll
       for (int cb = 0; cb < C::CBW; ++cb)
@@ -662,21 +665,21 @@ __device__ __forceinline__ void logits_stage(
     for (int mb = 0; mb < C::MBW; ++mb) {
       const u32x4 a = *reinterpret_cast<const u32x4*>(b + (arow0 + mb * 16) * 128 + rd[j]);
 #pragma unroll
-      for (int cb = 0; cb < C::CBW; ++cb)
-        acc[mb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8_r, a), __builtin_bit_cast(bf16x8_r, bf[cb]), acc[mb][cb], 0,
-            0, 0);
+      for (int cb = 0; cb < PL * C::CBW; ++cb)
+        acc[mb][cb % C::CBW] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8_r, a), __builtin_bit_cast(bf16x8_r, bf[cb]),
+            acc[mb][cb % C::CBW], 0, 0, 0);
     }
   }
 }
 
-template <int BT, int BE, int WM, int WN, int NB, bool ACC, bool WNORM>
+template <int BT, int BE, int WM, int WN, int NB, int PL, bool WNORM>
 __device__ __forceinline__ void router_logits_body(const DecodeArgs& p, float* wnorm,
                                                    uint16_t* __restrict__ s0,
                                                    uint16_t* __restrict__ s1,
                                                    uint16_t* __restrict__ s2,
                                                    uint16_t* __restrict__ s3) {
-  using C = LogitsTile<BT, BE, WM, WN>;
+  using C = LogitsTile<BT, BE, WM, WN, PL>;
   uint16_t* const sb[4] = {s0, s1, s2, s3};
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -688,7 +691,7 @@ __device__ __forceinline__ void router_logits_body(const DecodeArgs& p, float* w
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(p.x + (size_t)t0 * H), (short)0, trows * H * 2, 0x00020000);
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(p.router_w + (size_t)e0 * H), (short)0, BE * H * 2, 0x00020000);
+      (void*)(p.router_w + (size_t)e0 * H), (short)0, ((PL - 1) * p.E + BE) * H * 2, 0x00020000);
   // DMA ii of this wave covers stage rows 8 i .. 8 i + 7, i = wave + WAVES ii:
   // lane l fetches the slot that belongs at position l & 7 of row 8 i + l / 8
   uint32_t src[C::ND];
@@ -697,7 +700,10 @@ __device__ __forceinline__ void router_logits_body(const DecodeArgs& p, float* w
     const int i = wave + C::WAVES * ii;
     const int r = 8 * i + (lane >> 3);
     const int sl = (lane & 7) ^ stage_swizzle(r);
-    const int row = 8 * i >= BT ? r - BT : min(r, trows - 1);  // tokens past the end: the last
+    // tokens past the end: the last; then the router rows, plane by plane
+    const int row = 8 * i >= BT + BE ? r - BT - BE + p.E
+                    : 8 * i >= BT    ? r - BT
+                                     : min(r, trows - 1);
     src[ii] = ((uint32_t)row * H + sl * 8) * 2;
   }
   const int wm = wave % WM, wn = wave / WM;
@@ -742,7 +748,7 @@ __device__ __forceinline__ void router_logits_body(const DecodeArgs& p, float* w
         __builtin_amdgcn_sched_barrier(0);
         dma(sb[(q + NB - 1) % NB], min(c + q + NB - 1, nst - 1));
         __builtin_amdgcn_sched_barrier(0);
-        logits_stage<BT, BE, WM, WN, WNORM>(sb[q], rd, arow0, brow0, acc, ss, norms);
+        logits_stage<BT, BE, WM, WN, PL, WNORM>(sb[q], rd, arow0, brow0, acc, ss, norms);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(C::vmcnt((NB - 2) * C::ND));
         __builtin_amdgcn_s_barrier();
@@ -770,23 +776,22 @@ __device__ __forceinline__ void router_logits_body(const DecodeArgs& p, float* w
       for (int i = 0; i < 4; ++i) {
         const int t = t0 + arow0 + mb * 16 + 4 * kg + i;
         if (t < p.T) {
-          float* o = p.logits + ((size_t)blockIdx.z * p.T + t) * (p.E + 1) + e;
-          *o = ACC ? *o + acc[mb][cb][i] : acc[mb][cb][i];
+          p.logits[((size_t)blockIdx.z * p.T + t) * (p.E + 1) + e] = acc[mb][cb][i];
         }
       }
     }
 }
 
-template <int BT, int BE, int WM, int WN, int NB, bool ACC, bool WNORM>
+template <int BT, int BE, int WM, int WN, int NB, int PL, bool WNORM>
 __global__ __launch_bounds__(64 * WM * WN) void router_logits_kernel(const DecodeArgs p,
                                                                      float* wnorm) {
   static_assert(NB >= 3 && NB <= 4, "stage buffers");
-  using C = LogitsTile<BT, BE, WM, WN>;
+  using C = LogitsTile<BT, BE, WM, WN, PL>;
   __shared__ __attribute__((aligned(16))) uint16_t s0[C::ROWS * 64];
   __shared__ __attribute__((aligned(16))) uint16_t s1[C::ROWS * 64];
   __shared__ __attribute__((aligned(16))) uint16_t s2[C::ROWS * 64];
   __shared__ __attribute__((aligned(16))) uint16_t s3[NB > 3 ? C::ROWS * 64 : 8];
-  router_logits_body<BT, BE, WM, WN, NB, ACC, WNORM>(p, wnorm, s0, s1, s2, s3);
+  router_logits_body<BT, BE, WM, WN, NB, PL, WNORM>(p, wnorm, s0, s1, s2, s3);
 }
 
 __device__ __forceinline__ uint32_t f32_order_key(float v) {
@@ -1919,7 +1924,8 @@ bool router_mfma_eligible(int E, int H) {
 }
 
 // Tokens up to which the exact router in one launch beats logits and
-// selection (two launches, five with an 8-bit gate: split, both planes):
+// selection (two launches, three with an 8-bit gate, whose weights are split;
+// its columns below are from when each plane took a launch of its own):
 // whole block in us, matrix-core router against router_kernel, 4 bits, at
 // hidden 2048 | 1024 | 4096 (256 | 128 | 64 experts).
 //   8-bit gate: 16 tokens 88.8 -> 66.8 | 49.4 -> 37.5 | 92.5 -> 70.6;
@@ -1935,10 +1941,12 @@ int router_direct_tokens(bool rq8) { return rq8 ? 96 : 24; }
 // 11.7 against 17.3 us, at 8192 tokens 21.2 against 32.2 (event-timed).
 // The selection: a workgroup per token while the tokens number at most the
 // device's 1024 SIMDs (the re-checks of a token then run on four waves),
-// else a wave per token.
+// else a wave per token.  An 8-bit gate's re-checks are longer and the line
+// lies at twice that (1750 tokens: 26.6 -> 24.1 us; bf16 gate 1750 tokens:
+// block 247 against 249).
 template <int RQ, int XC>
 static void select_launch(const DecodeArgs& a, const void* wnorm, hipStream_t s) {
-  if (a.T <= 1024)
+  if (a.T <= (RQ ? 2048 : 1024))
     hipLaunchKernelGGL((router_select_kernel<RQ, XC, 4>), dim3(a.T), dim3(256), 0, s, a,
                        (const float*)wnorm);
   else
@@ -1946,14 +1954,14 @@ static void select_launch(const DecodeArgs& a, const void* wnorm, hipStream_t s)
                        a, (const float*)wnorm);
 }
 
-template <bool ACC, bool WNORM>
+template <int PL, bool WNORM>
 static void launch_logits(const DecodeArgs& a, float* wnorm, hipStream_t s) {
   const unsigned z = (unsigned)max(a.logit_planes, 1);
   if (a.T >= 4096)
-    hipLaunchKernelGGL((router_logits_kernel<64, 64, 2, 2, 3, ACC, WNORM>),
+    hipLaunchKernelGGL((router_logits_kernel<64, 64, 2, 2, 3, PL, WNORM>),
                        dim3((a.T + 63) / 64, a.E / 64, z), dim3(256), 0, s, a, wnorm);
   else
-    hipLaunchKernelGGL((router_logits_kernel<32, 32, 2, 2, 4, ACC, WNORM>),
+    hipLaunchKernelGGL((router_logits_kernel<32, 32, 2, 2, 4, PL, WNORM>),
                        dim3((a.T + 31) / 32, a.E / 32, z), dim3(256), 0, s, a, wnorm);
 }
 
@@ -1970,21 +1978,19 @@ int router_logit_planes(int T) {
 hipError_t launch_router_mfma(const DecodeArgs& a, float* wnorm, uint16_t* split,
                               hipStream_t s) {
   if (a.rq8) {
-    // logits over the hi plane, then continued over the lo plane
+    // logits over both planes at once
     hipLaunchKernelGGL(router_split_kernel, dim3((a.E + 3) / 4), dim3(256), 0, s, a, split,
                        split + (size_t)a.E * a.H, wnorm);
-    DecodeArgs hi = a, lo = a;
-    hi.router_w = split;
-    lo.router_w = split + (size_t)a.E * a.H;
-    launch_logits<false, false>(hi, nullptr, s);
-    launch_logits<true, false>(lo, nullptr, s);
+    DecodeArgs planes = a;
+    planes.router_w = split;
+    launch_logits<2, false>(planes, nullptr, s);
     if (a.H <= 2048)
       select_launch<1, 4>(a, wnorm, s);
     else
       select_launch<1, 8>(a, wnorm, s);
   } else {
     // the row norms come from the first token tile's workgroups
-    launch_logits<false, true>(a, wnorm, s);
+    launch_logits<1, true>(a, wnorm, s);
     if (a.H <= 2048)
       select_launch<0, 4>(a, wnorm, s);
     else

@@ -1303,11 +1303,22 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillArgs 
 }
 
 // --------------------------------------------------------------- launchers
-int prefill_tile_rows(int T, int K, int E) {
-  // few rows per expert (a short prefill chunk): 32-row tiles keep the
-  // wasted MFMA rows low; otherwise 128-row tiles share each dequantised
-  // weight fragment across more rows
-  return (long)T * K <= 48L * E ? 32 : kPrefillBM;
+// 32-row tiles waste few MFMA rows and spread few rows per expert over many
+// workgroups; 128-row tiles share each dequantised weight fragment across
+// more rows and pay once their workgroups fill the device.  R = rows per
+// expert on average; whole block in us, 32- against 128-row tiles, 8 bits |
+// 4 bits:
+//   hidden 2048, 256 experts: R 24 243/253 | 182/185, 32 281/270 | 217/208,
+//     48 351/293 | 272/239
+//   4096, 64 experts: R 44 215/207 | 161/166, 52 231/218 | 172/177,
+//     72 286/234 | 216/208
+//   1024, 128 experts: R 48 85/85 | 75/81, 64 94/91 | 85/88, 96 111/103 | 99/101
+//   512, 32 experts: R 72 43/56 | 41/55, 128 57/67 | 55/67
+// so 128 rows from R = 30 on if a call has `enough` 32-row gate/up tiles.
+int prefill_tile_rows(int T, int K, int E, int H, int I, int bits) {
+  const long rows = (long)T * K;
+  const long enough = bits == 4 && H <= 1024 ? 1500 : 800;  // (1024 x 4 bits: R 91)
+  return rows <= 30L * E || rows / 32 * (I / 64) <= enough ? 32 : kPrefillBM;
 }
 
 int prefill_sort_slices(int T, int K) {
@@ -1393,7 +1404,7 @@ bool buffer_offsets_fit(const PrefillArgs& a, int bits) {
 
 hipError_t launch_prefill(const PrefillArgs& args, int bits, bool combine, hipStream_t s) {
   PrefillArgs a = args;
-  a.bm = prefill_tile_rows(a.T, a.K, a.E);
+  a.bm = prefill_tile_rows(a.T, a.K, a.E, a.H, a.I, bits);
   if (a.bm == kPrefillBM && !buffer_offsets_fit(a, bits)) return hipErrorInvalidValue;
   const int nw = prefill_sort_slices(a.T, a.K);
   // one slice: the place kernel counts its rows itself

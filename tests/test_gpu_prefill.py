@@ -257,3 +257,18 @@ def test_long_prefill_skewed_routing_4bit(torch_cuda):
     mx_ = M.bf16_to_f32(mlx)
     assert np.abs(got - mx_).max() <= MAX_ABS
     assert cosine(got.reshape(-1), mx_.reshape(-1)) >= MIN_COS
+
+
+@pytest.mark.parametrize("bits,T", [(8, 800), (8, 808), (4, 1496), (4, 1504)])
+def test_tile_height_rule(torch_cuda, bits, T):
+    """Either side of the work at which a call takes 128-row tiles (800
+    32-row gate/up tiles, 1500 at 4 bits and hidden up to 1024; 8 experts of
+    intermediate 512, so rows per expert are far past the other condition)."""
+    L = M.make_layer(77 + bits, hidden=256, inter=512, experts=8, top_k=4, bits=bits,
+                     shared=False)
+    x = M.make_x(7 + T, T, 256)
+    idx = np.random.default_rng(T).integers(0, 8, size=(T, 4)).astype(np.int32)
+    got = _switch(torch_cuda, L, x, idx)
+    ref = M.switch_glu(L, x, idx, mode="prefill")
+    assert _mismatches(got, ref) <= got.size // 500
+    assert cosine(got.reshape(-1), ref.reshape(-1)) >= MIN_COS

@@ -131,6 +131,22 @@ int rmoe_abi_version(void);
  * aligned. */
 int rmoe_rms_norm(const uint16_t* x, const uint16_t* weight, int32_t tokens, int32_t hidden,
                   float eps, uint16_t* out, void* stream);
+/* out[t] = bf16(sum_j weights[t, j] y[t, j] + sigmoid(gate[t]) shared[t]) in
+ * fp32, the slots in order, then the shared expert's row; with a residual
+ * bf16(residual[t] + that).  The tail of mlx-lm's block around a SwitchGLU
+ * (bench/mlx_lm_adapter.py:49-94) for rows that are already computed.
+ * y bf16 [tokens, top_k, hidden], weights fp32 [tokens, top_k], shared bf16
+ * [tokens, hidden] with its gate's logits bf16 [tokens], or both NULL;
+ * hidden a multiple of 8; row arrays 16-byte aligned. */
+int rmoe_combine(const uint16_t* y, const float* weights, int32_t tokens, int32_t top_k,
+                 int32_t hidden, const uint16_t* shared, const uint16_t* gate,
+                 const uint16_t* residual, uint16_t* out, void* stream);
+
+/* out = bf16(bf16(silu(gate)) * up) over n bf16 values (mlx-lm SwiGLU on
+ * separate projections); 16-byte aligned. */
+int rmoe_swiglu(const uint16_t* up, const uint16_t* gate, int64_t n, uint16_t* out,
+                void* stream);
+
 const char* rmoe_last_error(void);
 const char* rmoe_status_string(int status);
 

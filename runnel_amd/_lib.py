@@ -33,7 +33,7 @@ EXPORTED = (
     "rmoe_router_workspace_bytes", "rmoe_chain_table_bytes", "rmoe_chain_table_pack",
     "rmoe_moe_chain", "rmoe_workspace_status_offset", "rmoe_router_q",
     "rmoe_switch_combine", "rmoe_switch_combine_workspace_bytes", "rmoe_rms_norm",
-    "rmoe_set_cooperative_launch", "rmoe_moe_block_noalloc",
+    "rmoe_set_cooperative_launch", "rmoe_moe_block_noalloc", "rmoe_combine", "rmoe_swiglu",
 )
 
 # rmoe_moe_block_noalloc's static scratch per GPU (RMOE_NOALLOC_SCRATCH_BYTES)
@@ -109,6 +109,8 @@ def load() -> ctypes.CDLL:
         lib.rmoe_router.argtypes = [P, I32, I32, I32, I32, P, I32, P, P, P, SZ, P]
         lib.rmoe_router_q.argtypes = [QP, I32, I32, P, I32, P, P, P, SZ, P]
         lib.rmoe_rms_norm.argtypes = [P, P, I32, I32, ctypes.c_float, P, P]
+        lib.rmoe_combine.argtypes = [P, P, I32, I32, I32, P, P, P, P, P]
+        lib.rmoe_swiglu.argtypes = [P, P, I64, P, P]
         lib.rmoe_router_workspace_bytes.restype = SZ
         lib.rmoe_router_workspace_bytes.argtypes = [I32, I32, I32]
         lib.rmoe_switch_glu.argtypes = [QP, QP, P, I32, P, I32, P, P, SZ, P]

@@ -617,6 +617,40 @@ int rmoe_rms_norm(const uint16_t* x, const uint16_t* weight, int32_t tokens, int
   return ok();
 }
 
+int rmoe_combine(const uint16_t* y, const float* weights, int32_t tokens, int32_t top_k,
+                 int32_t hidden, const uint16_t* shared, const uint16_t* gate,
+                 const uint16_t* residual, uint16_t* out, void* stream) {
+  if (tokens < 0) return fail(RMOE_EINVAL, "tokens must be >= 0 (got %d)", tokens);
+  if (top_k < 1) return fail(RMOE_EINVAL, "top_k must be >= 1 (got %d)", top_k);
+  if (hidden < 8 || hidden % 8 || hidden > 2048 * 65535)
+    return fail(RMOE_EINVAL, "hidden must be a positive multiple of 8 (got %d)", hidden);
+  if ((shared != nullptr) != (gate != nullptr))
+    return fail(RMOE_EINVAL, "shared and gate must be given together");
+  if (tokens == 0) return ok();
+  if (!y || !weights || !out) return fail(RMOE_ENULL, "y, weights and out are required");
+  if (!aligned(y, 16) || !aligned(out, 16) || !aligned(shared, 16) || !aligned(residual, 16) ||
+      !aligned(weights, 4) || !aligned(gate, 2))
+    return fail(RMOE_EALIGN, "row arrays must be 16-byte aligned");
+  const hipError_t e = rmoe::launch_combine(y, weights, tokens, top_k, hidden, shared, gate,
+                                            residual, out, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "combine launch");
+  return ok();
+}
+
+int rmoe_swiglu(const uint16_t* up, const uint16_t* gate, int64_t n, uint16_t* out,
+                void* stream) {
+  if (n < 0 || n > (int64_t)2048 * 0x7FFFFFFF / 256)
+    return fail(RMOE_EINVAL, "n out of range (got %lld)", (long long)n);
+  if (n == 0) return ok();
+  if (!up || !gate || !out) return fail(RMOE_ENULL, "up, gate and out are required");
+  if (!aligned(up, 16) || !aligned(gate, 16) || !aligned(out, 16))
+    return fail(RMOE_EALIGN, "up, gate and out must be 16-byte aligned");
+  const hipError_t e =
+      rmoe::launch_swiglu(up, gate, n, out, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "swiglu launch");
+  return ok();
+}
+
 int rmoe_router_q(const rmoe_qweight* router, int32_t top_k, int32_t norm_topk_prob,
                   const uint16_t* x, int32_t tokens, int32_t* indices, float* scores,
                   void* ws, size_t ws_bytes, void* stream) {

@@ -134,6 +134,13 @@ hipError_t launch_router(const DecodeArgs& a, hipStream_t s);
 // RMSNorm of T rows of H bf16 values (H a multiple of 8; x, w, out 16-byte aligned).
 hipError_t launch_rmsnorm(const uint16_t* x, const uint16_t* w, int T, int H, float eps,
                           uint16_t* out, hipStream_t s);
+// The tail of a block whose rows are computed apart: weighted sum of the
+// slots, gated shared row (or null), residual (or null).
+hipError_t launch_combine(const uint16_t* y, const float* w, int T, int K, int H,
+                          const uint16_t* shared, const uint16_t* gate, const uint16_t* residual,
+                          uint16_t* out, hipStream_t s);
+hipError_t launch_swiglu(const uint16_t* up, const uint16_t* gate, int64_t n, uint16_t* out,
+                         hipStream_t s);
 // Many-token router on the matrix cores with exact selection (prefill).
 bool router_mfma_eligible(int E, int H);
 int router_direct_tokens(bool rq8);  // up to this many tokens launch_router is faster

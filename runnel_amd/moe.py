@@ -248,11 +248,18 @@ class SparseMoeBlock(nn.Module):
             raise ValueError("router gate must be bf16 or 8-bit group-64 affine")
         inds, scores = native.router(router, x2, self.top_k, self.norm_topk_prob)
         y = self.switch_mlp(x2, inds)  # [T, k, D]
-        out = (y.float() * scores[..., None]).sum(dim=-2)
+        sh = sg = None
         if self.shared_expert is not None:
-            sh = self.shared_expert(x2).float()
-            sg = torch.sigmoid(self.shared_expert_gate(x2).float())
-            out = out + sg * sh
+            sh, sg = self.shared_expert(x2), self.shared_expert_gate(x2)
+        res = None if residual is None else residual.reshape(-1, D)
+        rows = [t for t in (y, sh, res) if t is not None]
+        if (native.rows_ready(*rows) and y.dim() == 3 and D % 8 == 0
+                and (sg is None or (sg.dtype == BF16 and tuple(sg.shape) == (len(x2), 1)
+                                    and not sg.requires_grad))):
+            return native.combine(y, scores, sh, sg, res).reshape(*lead, D)
+        out = (y.float() * scores[..., None]).sum(dim=-2)
+        if sh is not None:
+            out = out + torch.sigmoid(sg.float()) * sh.float()
         out = out.to(BF16)
         if residual is not None:
             out = (residual.reshape(-1, D).float() + out.float()).to(BF16)

@@ -563,6 +563,58 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.
     return out.reshape(x.shape)
 
 
+def rows_ready(*tensors) -> bool:
+    """Whether every tensor is a contiguous, 16-byte aligned bf16 GPU tensor
+    outside autograd: what the row kernels below take as it is."""
+    return all(t.dtype == BF16 and t.is_cuda and t.is_contiguous() and not t.requires_grad
+               and t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def combine(y: torch.Tensor, weights: torch.Tensor, shared: torch.Tensor | None = None,
+            gate: torch.Tensor | None = None,
+            residual: torch.Tensor | None = None) -> torch.Tensor:
+    """bf16(sum_j weights[t, j] y[t, j] + sigmoid(gate[t]) shared[t]) of rows y
+    bf16 [T, k, H] (fp32 sums, slots in order), then + residual in bf16:
+    weights float32 [T, k], shared bf16 [T, H] with gate logits bf16 [T] or
+    both None -> bf16 [T, H]."""
+    lib = _lib.load()
+    if y.dtype != BF16 or y.dim() != 3:
+        raise ValueError("y must be a bfloat16 [tokens, k, hidden] tensor")
+    T, k, H = y.shape
+    if weights.dtype != torch.float32 or tuple(weights.shape) != (T, k):
+        raise ValueError(f"weights must be float32 [{T}, {k}] (got {list(weights.shape)})")
+    if (shared is None) != (gate is None):
+        raise ValueError("shared and gate must be given together")
+    if shared is not None:
+        _check_rows(shared, "shared", T, H)
+        if gate.dtype != BF16 or gate.numel() != T:
+            raise ValueError(f"gate must be {T} bfloat16 logits (got {list(gate.shape)})")
+        shared, gate = shared.contiguous(), gate.contiguous()
+    if residual is not None:
+        _check_rows(residual, "residual", T, H)
+        residual = residual.contiguous()
+    _require_cuda(y, weights, shared, gate, residual)
+    y, weights = y.contiguous(), weights.contiguous()
+    out = torch.empty((T, H), dtype=BF16, device=y.device)
+    _lib.check(lib.rmoe_combine(y.data_ptr(), weights.data_ptr(), T, k, H, _lib.ptr(shared),
+                                _lib.ptr(gate), _lib.ptr(residual), out.data_ptr(),
+                                _lib.stream_handle(y.device)))
+    return out
+
+
+def swiglu(up: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
+    """bf16(bf16(silu(gate)) * up) of two bf16 tensors of one shape."""
+    lib = _lib.load()
+    if up.dtype != BF16 or gate.dtype != BF16 or up.shape != gate.shape:
+        raise ValueError("up and gate must be bfloat16 of one shape")
+    _require_cuda(up, gate)
+    up, gate = up.contiguous(), gate.contiguous()
+    out = torch.empty_like(up)
+    _lib.check(lib.rmoe_swiglu(up.data_ptr(), gate.data_ptr(), up.numel(), out.data_ptr(),
+                               _lib.stream_handle(up.device)))
+    return out
+
+
 def quantize(w: torch.Tensor, bits: int, group_size: int = 64):
     """Affine quantization of float32 [..., K] on the GPU ->
     (int32 words [..., K*bits/32], bf16 scales, bf16 biases)."""

@@ -111,6 +111,19 @@ class QuantizedLinear(_Params):
         return y.reshape(*lead, self.output_dims)
 
 
+def _x_rows(x, indices):
+    """Row of x [..., 1 or k, 1, in] that each index [..., k] takes, as int32;
+    None where they pair one to one."""
+    xb = x.shape[:-2]
+    if tuple(xb) == tuple(indices.shape):
+        return None
+    n_x = 1
+    for d in xb:
+        n_x *= d
+    lhs = torch.arange(n_x, device=x.device, dtype=torch.int32).reshape(xb)
+    return torch.broadcast_to(lhs, indices.shape).reshape(-1)
+
+
 class QuantizedSwitchLinear(_Params):
     """Expert bank [num_experts, out, in] in MLX-affine format with mlx-lm's
     call convention: ``__call__(x, indices, sorted_indices=False)`` where x
@@ -162,15 +175,12 @@ class QuantizedSwitchLinear(_Params):
         del sorted_indices  # row order does not change any result here
         if self.mode != "affine":
             raise ValueError(f"quantization mode {self.mode!r} is not supported")
-        D = x.shape[-1]
+        return self._gather(x, indices, _x_rows(x, indices))
+
+    def _gather(self, x, indices, lhs):
+        """The product for x rows `lhs` (as _x_rows gives them)."""
         idx_shape = indices.shape
-        xb = x.shape[:-2]
-        n_x = 1
-        for d in xb:
-            n_x *= d
-        lhs = torch.arange(n_x, device=x.device, dtype=torch.int32).reshape(xb)
-        lhs = torch.broadcast_to(lhs, idx_shape).reshape(-1)
-        y = native.gather_qmm(x.reshape(n_x, D), self.weight, self.scales, self.biases,
+        y = native.gather_qmm(x.reshape(-1, x.shape[-1]), self.weight, self.scales, self.biases,
                               self.bits, self.group_size,
                               rhs_indices=indices.reshape(-1), lhs_indices=lhs)
         if "bias" in self:
@@ -182,12 +192,23 @@ def swiglu(x: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.silu(gate) * x
 
 
+def _activate(activation, x, gate):
+    """activation(x, gate); the package's own SwiGLU of two kernel outputs in
+    one launch."""
+    if type(activation) is SwiGLU and x.shape == gate.shape and native.rows_ready(x, gate):
+        return native.swiglu(x, gate)
+    return activation(x, gate)
+
+
 class SwiGLU(nn.Module):
     """mlx-lm ``SwiGLU``: ``activation(x_up, x_gate) = silu(x_gate) * x_up``
     (called as at src/runnel/mlx.py:78)."""
 
     def __call__(self, x, gate):
         return swiglu(x, gate)
+
+
+_SWIGLU = SwiGLU()
 
 
 class SwitchGLU(nn.Module):
@@ -208,9 +229,13 @@ class SwitchGLU(nn.Module):
 
     def __call__(self, x, indices):
         x = x.unsqueeze(-2).unsqueeze(-3)  # expand_dims(x, (-2, -3))
-        x_up = self.up_proj(x, indices)
-        x_gate = self.gate_proj(x, indices)
-        x = self.down_proj(self.activation(x_up, x_gate), indices)
+        up, gate = self.up_proj, self.gate_proj
+        if all(type(p) is QuantizedSwitchLinear and p.mode == "affine" for p in (up, gate)):
+            lhs = _x_rows(x, indices)  # once for both
+            x_up, x_gate = up._gather(x, indices, lhs), gate._gather(x, indices, lhs)
+        else:
+            x_up, x_gate = up(x, indices), gate(x, indices)
+        x = self.down_proj(_activate(self.activation, x_up, x_gate), indices)
         return x.squeeze(-2)
 
 
@@ -225,4 +250,4 @@ class MLP(nn.Module):
         self.down_proj = QuantizedLinear(hidden_dim, dim, bits, group_size, device=device)
 
     def __call__(self, x):
-        return self.down_proj(swiglu(self.up_proj(x), self.gate_proj(x)))
+        return self.down_proj(_activate(_SWIGLU, self.up_proj(x), self.gate_proj(x)))

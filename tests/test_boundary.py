@@ -552,3 +552,17 @@ def test_noalloc_block_refuses_calls_beyond_its_static_scratch():
                                       FAKE + 2, None) == _lib.RMOE_EALIGN
     assert lib.rmoe_moe_block_noalloc(ctypes.byref(L), FAKE, 0, None, FAKE + 4096, None, None,
                                       None, None) == _lib.RMOE_OK
+
+
+def test_combine_and_swiglu_reject_before_launch():
+    lib = _lib.load()
+    combine, ok = lib.rmoe_combine, _lib.RMOE_OK
+    assert combine(FAKE, FAKE, 3, 0, 64, None, None, None, FAKE, None) == _lib.RMOE_EINVAL
+    assert combine(FAKE, FAKE, 3, 2, 60, None, None, None, FAKE, None) == _lib.RMOE_EINVAL
+    assert combine(FAKE, FAKE, 3, 2, 64, FAKE, None, None, FAKE, None) == _lib.RMOE_EINVAL
+    assert combine(FAKE, None, 3, 2, 64, None, None, None, FAKE, None) == _lib.RMOE_ENULL
+    assert combine(FAKE + 2, FAKE, 3, 2, 64, None, None, None, FAKE, None) == _lib.RMOE_EALIGN
+    assert combine(None, None, 0, 2, 64, None, None, None, None, None) == ok
+    assert lib.rmoe_swiglu(FAKE, FAKE, -1, FAKE, None) == _lib.RMOE_EINVAL
+    assert lib.rmoe_swiglu(FAKE, FAKE + 2, 8, FAKE, None) == _lib.RMOE_EALIGN
+    assert lib.rmoe_swiglu(None, None, 0, None, None) == ok

@@ -497,6 +497,7 @@ int switch_call(const rmoe_qweight* gate_up, const rmoe_qweight* down, const uin
       top_k <= rmoe::kMaxFusedRouted && H == rmoe::kFusedH && I == rmoe::kFusedI &&
       aligned(gate_up->scales, 4) && aligned(gate_up->biases, 4))
     a.few_bits = gate_up->bits;
+  a.act16 = a.few_bits == 0 && rmoe::down_few_ok(tokens, top_k, I);
   hipError_t e = rmoe::launch_gate_up(a, gate_up->bits, s);
   if (e != hipSuccess) return hip_fail(e, "gate/up launch");
   e = rmoe::launch_down(a, gate_up->bits, combine, s);
@@ -767,6 +768,7 @@ int block_launch(const rmoe_layer* L, const uint16_t* x, int32_t tokens,
     if (e != hipSuccess) return hip_fail(e, "prefill launch");
     return ok();
   }
+  a.act16 = a.few_bits == 0 && rmoe::down_few_ok(tokens, a.K + a.has_shared, a.I);
   e = rmoe::launch_gate_up(a, bits, s);
   if (e != hipSuccess) return hip_fail(e, "gate/up launch");
   e = rmoe::launch_down(a, bits, true, s);

@@ -1219,7 +1219,13 @@ __global__ __launch_bounds__(256) void gate_up_kernel(const DecodeArgs p,
   if (!shared && (unsigned)e >= (unsigned)p.E) {
     // Caller index outside the bank: the slot contributes zeros and no
     // weight memory is touched.
-    if (lane < PPW && c0 + lane < I) p.act[(size_t)unit * I + c0 + lane] = 0.0f;
+    if (lane < PPW && c0 + lane < I) {
+      const size_t at = (size_t)unit * I + c0 + lane;
+      if (p.act16)
+        reinterpret_cast<uint16_t*>(p.act)[at] = 0;
+      else
+        p.act[at] = 0.0f;
+    }
     return;
   }
   const int H = p.H;
@@ -1293,7 +1299,11 @@ __global__ __launch_bounds__(256) void gate_up_kernel(const DecodeArgs p,
     if (lane == 0) {
       const float up = round_bf16(au);
       const float gate = round_bf16(ag);
-      p.act[(size_t)unit * I + c] = round_bf16(silu(gate) * up);
+      const uint32_t a = f32_to_bf16(silu(gate) * up);
+      if (p.act16)
+        reinterpret_cast<uint16_t*>(p.act)[(size_t)unit * I + c] = (uint16_t)a;
+      else
+        p.act[(size_t)unit * I + c] = bf16_to_f32(a);
     }
   }
 }
@@ -1539,15 +1549,16 @@ __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
 // rows meet in LDS and lanes 0 .. R - 1 sum them in slot order (weighted),
 // then the residual; otherwise each wave writes its per-slot rows y[t, j, h].
 // R = 16 rows up to 4 tokens, 8 beyond (more, shorter workgroups).
-template <int BITS, bool COMBINE, int R>
+// I = 128, 256 and 512 (fewer lanes a row, more rows a pass); H a multiple of R.
+template <int BITS, bool COMBINE, int I, int R>
 __global__ __launch_bounds__(64 * kMaxFusedUnits) void down_few_kernel(const DecodeArgs p) {
-  constexpr int H = few::H;
-  constexpr int I = few::I;
+  const int H = p.H;
   constexpr int NU = kMaxFusedUnits;
-  constexpr int LPR = BITS == 8 ? 32 : 16;  // lanes per row
-  constexpr int RPW = 64 / LPR;             // rows per pass: 2 | 4
-  constexpr int RP = R / RPW;               // passes
   constexpr int VPL = BITS == 8 ? 16 : 32;  // values per lane
+  constexpr int LPR = I / VPL;              // lanes per row (I 512: 32 | 16)
+  constexpr int RPW = 64 / LPR;             // rows per pass (2 | 4)
+  constexpr int RP = R / RPW;               // passes
+  static_assert(R % RPW == 0, "whole passes");
   constexpr int WPR = I * BITS / 32;        // words per down row
   constexpr int GD = I / 64;                // groups per down row
   constexpr int AV = VPL / 8;               // 16-byte activation pieces per lane
@@ -2146,6 +2157,19 @@ static hipError_t gate_up_cpl(const DecodeArgs& a, hipStream_t s) {
   return hipSuccess;
 }
 
+// Calls below the expert-sorted threshold, any hidden size.  Against
+// down_kernel, block / switch call in us, 8 bits:
+//   hidden 1024, intermediate 256, 8 slots: 1 token 19.2/13.8 -> 14.1/8.0,
+//     4 24.7/15.9 -> 18.0/10.2, 7 27.8/19.4 -> 21.3/13.5
+//   4096, 512, 4 slots: 1 25.4/17.3 -> 21.2/14.0, 8 94.7/69.6 -> 76.5/53.6,
+//     15 164/124 -> 126/92
+//   512, 128, 4 slots: 1 15.3/9.9 -> 11.8/6.8, 15 18.8/11.6 -> 16.1/8.4
+// (4 bits: 1 token at 1024 22.7/16.1 -> 14.8/8.2, at 512 17.2/11.4 -> 12.4/7.3;
+// 8 tokens at 4096 61.4/44.1 -> 54.2/36.3).
+bool down_few_ok(int T, int units, int I) {
+  return T <= kPrefillMinRows && units <= kMaxFusedUnits && (I == 128 || I == 256 || I == 512);
+}
+
 hipError_t launch_gate_up(const DecodeArgs& a, int bits, hipStream_t s) {
   if (a.few_bits != 0) {
     const int waves = a.T * a.K * few::kWavesPerUnit;
@@ -2170,29 +2194,35 @@ hipError_t launch_gate_up(const DecodeArgs& a, int bits, hipStream_t s) {
 }
 
 hipError_t launch_down(const DecodeArgs& a, int bits, bool combine, hipStream_t s) {
-  if (a.few_bits != 0) {
-    // rows per workgroup: 16 up to 4 tokens, 8 beyond
-    const dim3 block(64 * kMaxFusedUnits);
-    auto go = [&](auto bits_c, auto combine_c, auto r_c) {
+  if (a.few_bits != 0 || a.act16) {
+    // rows per workgroup: 16 up to 4 tokens, 8 beyond (16 where a pass of
+    // the wave is that many)
+    auto go = [&](auto bits_c, auto combine_c, auto i_c) {
       constexpr int B = decltype(bits_c)::value;
       constexpr bool C = decltype(combine_c)::value;
-      constexpr int R = decltype(r_c)::value;
-      hipLaunchKernelGGL((down_few_kernel<B, C, R>), dim3((unsigned)(a.T * (few::H / R))), block,
-                         0, s, a);
+      constexpr int I = decltype(i_c)::value;
+      constexpr int RS = B == 4 && I == 128 ? 16 : 8;
+      const dim3 block(64 * kMaxFusedUnits);
+      if (a.T <= 4)
+        hipLaunchKernelGGL((down_few_kernel<B, C, I, 16>), dim3((unsigned)(a.T * (a.H / 16))),
+                           block, 0, s, a);
+      else
+        hipLaunchKernelGGL((down_few_kernel<B, C, I, RS>), dim3((unsigned)(a.T * (a.H / RS))),
+                           block, 0, s, a);
+    };
+    auto width = [&](auto bits_c, auto combine_c) {
+      if (a.I == 512) go(bits_c, combine_c, std::integral_constant<int, 512>{});
+      else if (a.I == 256) go(bits_c, combine_c, std::integral_constant<int, 256>{});
+      else go(bits_c, combine_c, std::integral_constant<int, 128>{});
     };
     using B8 = std::integral_constant<int, 8>;
     using B4 = std::integral_constant<int, 4>;
-    using CT = std::true_type;
-    using CF = std::false_type;
-    using R16 = std::integral_constant<int, 16>;
-    using R8 = std::integral_constant<int, 8>;
-    const bool wide = a.T <= 4;
-    if (a.few_bits == 8) {
-      if (combine) wide ? go(B8{}, CT{}, R16{}) : go(B8{}, CT{}, R8{});
-      else wide ? go(B8{}, CF{}, R16{}) : go(B8{}, CF{}, R8{});
+    if (bits == 8) {
+      if (combine) width(B8{}, std::true_type{});
+      else width(B8{}, std::false_type{});
     } else {
-      if (combine) wide ? go(B4{}, CT{}, R16{}) : go(B4{}, CT{}, R8{});
-      else wide ? go(B4{}, CF{}, R16{}) : go(B4{}, CF{}, R8{});
+      if (combine) width(B4{}, std::true_type{});
+      else width(B4{}, std::false_type{});
     }
     RMOE_CHECK_LAUNCH();
     return hipSuccess;

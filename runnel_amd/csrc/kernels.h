@@ -45,6 +45,8 @@ struct DecodeArgs {
   int few_bits;      // 8 | 4: the few-token kernels at these bits (act is
                      // bf16; the router launch also computes the shared
                      // expert's gate/up); 0: the general kernels
+  int act16;         // 1: the general gate/up writes act as bf16 for the
+                     // few-token down kernel (few_bits == 0)
   uint16_t* out;     // [T, H] (block) or [T, K, H] (switch)
   const uint16_t* residual;
   int32_t* idx_out;
@@ -148,6 +150,8 @@ int router_logit_planes(int T);
 // wnorm: [E] floats; split: [2, E, H] bf16 (quantized gates only)
 hipError_t launch_router_mfma(const DecodeArgs& a, float* wnorm, uint16_t* split,
                               hipStream_t s);
+// Calls of few tokens whose down projection the few-token kernel takes.
+bool down_few_ok(int T, int units, int I);
 hipError_t launch_gate_up(const DecodeArgs& a, int bits, hipStream_t s);
 hipError_t launch_down(const DecodeArgs& a, int bits, bool combine, hipStream_t s);
 hipError_t launch_qmv(const QmvArgs& a, int bits, hipStream_t s);

@@ -161,3 +161,34 @@ def test_few_token_switch(torch_cuda, bits, T, k):
     exp = M.round_bf16((rows * w[..., None]).sum(1).astype(np.float32))
     exp = M.f32_to_bf16(M.bf16_to_f32(res) + exp)
     _check(host_bf16(out), exp, exp)
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("H,I,T,k,shared", [
+    (64, 128, 1, 8, True), (192, 128, 5, 4, True), (512, 256, 4, 8, True),
+    (1024, 256, 7, 8, False), (320, 512, 15, 4, True), (128, 128, 63, 1, True),
+    (256, 64, 3, 4, True), (256, 256, 3, 9, True)])  # the last two: the general kernel
+def test_few_token_down_widths(torch_cuda, bits, H, I, T, k, shared):
+    """The down kernel's intermediate sizes and rows per workgroup (16 up to
+    4 tokens, 8 beyond), blocks and per-slot rows with ids outside the bank.
+    Same bounds as the block above."""
+    torch = torch_cuda
+    from helpers import bank_to_dev, dev_i32
+    from runnel_amd import native
+    print(f"few-token down bits={bits} H={H} I={I} T={T} k={k}", flush=True)
+    L = M.make_layer(700 + H + I + T, hidden=H, inter=I, experts=16, top_k=k, bits=bits,
+                     shared=shared)
+    x = M.make_x(60 + T, T, H)
+    out = native.moe_block(layer_to_dev(L), dev_bf16(x), residual=dev_bf16(x))
+    ref, mlx = (M.block_forward(L, x, residual_bits=x, mode=m)[0] for m in ("contract", "mlx"))
+    _check(host_bf16(out), ref, mlx)
+    idx = np.random.default_rng(T * k).integers(0, 16, (T, k)).astype(np.int32)
+    given = idx.copy()
+    given[T - 1, k - 1] = 16
+    keep = (bank_to_dev(L.gate_up), bank_to_dev(L.down))
+    y = native.switch_glu(dev_bf16(x), dev_i32(given),
+                          *(native.qweight_struct(*b, bits) for b in keep))
+    ref, mlx = (M.switch_glu(L, x, idx, mode=m) for m in ("contract", "mlx"))
+    ref[T - 1, k - 1] = mlx[T - 1, k - 1] = 0.0
+    _check(host_bf16(y), M.f32_to_bf16(ref), M.f32_to_bf16(mlx))
+    assert not host_bf16(y)[T - 1, k - 1].any()

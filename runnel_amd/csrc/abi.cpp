@@ -621,7 +621,8 @@ int rmoe_rms_norm(const uint16_t* x, const uint16_t* weight, int32_t tokens, int
 int rmoe_combine(const uint16_t* y, const float* weights, int32_t tokens, int32_t top_k,
                  int32_t hidden, const uint16_t* shared, const uint16_t* gate,
                  const uint16_t* residual, uint16_t* out, void* stream) {
-  if (tokens < 0) return fail(RMOE_EINVAL, "tokens must be >= 0 (got %d)", tokens);
+  int rc;
+  if ((rc = check_tokens(tokens))) return rc;
   if (top_k < 1) return fail(RMOE_EINVAL, "top_k must be >= 1 (got %d)", top_k);
   if (hidden < 8 || hidden % 8 || hidden > 2048 * 65535)
     return fail(RMOE_EINVAL, "hidden must be a positive multiple of 8 (got %d)", hidden);

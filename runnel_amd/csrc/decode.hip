@@ -1077,6 +1077,11 @@ void router_select_kernel(const DecodeArgs p, const float* wnorm) {
 // ..., then the butterfly), ms, v, r correctly rounded in fp32 (the library is
 // built with correctly rounded fp32 division and square root).  One wave
 // per token.
+// NC: pieces of 8 values per lane, all of them and their weights requested at
+// once and kept (H <= 512 NC); 0: any H, a loop for the sum and one for the
+// result.  Latency bound: the loops took 3.9, 5.1 and 7.5 us at 5, 61 and 1750 tokens
+// of 2048, one round trip takes 3.6, 4.7 and 6.4.
+template <int NC>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* x, const uint16_t* w,
                                                       int T, int H, float eps, uint16_t* out) {
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -1085,20 +1090,15 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* x, const u
   const uint16_t* xt = x + (size_t)t * H;
   const int chunks = H >> 3;
   float acc = 0.0f;
-  for (int c = lane; c < chunks; c += 64) {
-    const uint4 v = load16(xt + c * 8);
+  auto square = [&](const uint4 v) {
     const uint32_t vv[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       acc = fmaf(bf16_lo(vv[i]), bf16_lo(vv[i]), acc);
       acc = fmaf(bf16_hi(vv[i]), bf16_hi(vv[i]), acc);
     }
-  }
-  const float ms = wave_sum(acc) / (float)H;
-  const float r = 1.0f / sqrtf(ms + eps);
-  for (int c = lane; c < chunks; c += 64) {
-    const uint4 v = load16(xt + c * 8);
-    const uint4 g = load16(w + c * 8);
+  };
+  auto store = [&](int c, const uint4 v, const uint4 g, float r) {
     const uint32_t vv[4] = {v.x, v.y, v.z, v.w};
     const uint32_t gg[4] = {g.x, g.y, g.z, g.w};
     uint32_t o[4];
@@ -1109,6 +1109,33 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* x, const u
       o[i] = f32_to_bf16(lo) | (f32_to_bf16(hi) << 16);
     }
     *reinterpret_cast<uint4*>(out + (size_t)t * H + c * 8) = make_uint4(o[0], o[1], o[2], o[3]);
+  };
+  auto scale = [&] {
+    const float ms = wave_sum(acc) / (float)H;
+    return 1.0f / sqrtf(ms + eps);
+  };
+  if constexpr (NC > 0) {
+    uint4 v[NC], g[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int c = lane + 64 * i;
+      v[i] = g[i] = make_uint4(0, 0, 0, 0);
+      if (c < chunks) v[i] = load16(xt + c * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if (lane + 64 * i < chunks) g[i] = load16(w + (lane + 64 * i) * 8);
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if (lane + 64 * i < chunks) square(v[i]);
+    const float r = scale();
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if (lane + 64 * i < chunks) store(lane + 64 * i, v[i], g[i], r);
+  } else {
+    for (int c = lane; c < chunks; c += 64) square(load16(xt + c * 8));
+    const float r = scale();
+    for (int c = lane; c < chunks; c += 64) store(c, load16(xt + c * 8), load16(w + c * 8), r);
   }
 }
 
@@ -1549,10 +1576,12 @@ __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
 // rows meet in LDS and lanes 0 .. R - 1 sum them in slot order (weighted),
 // then the residual; otherwise each wave writes its per-slot rows y[t, j, h].
 // R = 16 rows up to 4 tokens, 8 beyond (more, shorter workgroups).
-// I = 128, 256 and 512 (fewer lanes a row, more rows a pass); H a multiple of R.
-template <int BITS, bool COMBINE, int I, int R>
+// I = 128, 256 and 512 (fewer lanes a row, more rows a pass); H_ = 0: any H, a
+// multiple of R (6 tokens at hidden 2048, 4 bits: 0.2 us per call more than
+// the constant).
+template <int BITS, bool COMBINE, int H_, int I, int R>
 __global__ __launch_bounds__(64 * kMaxFusedUnits) void down_few_kernel(const DecodeArgs p) {
-  const int H = p.H;
+  const int H = H_ ? H_ : p.H;
   constexpr int NU = kMaxFusedUnits;
   constexpr int VPL = BITS == 8 ? 16 : 32;  // values per lane
   constexpr int LPR = I / VPL;              // lanes per row (I 512: 32 | 16)
@@ -1567,8 +1596,10 @@ __global__ __launch_bounds__(64 * kMaxFusedUnits) void down_few_kernel(const Dec
   const int units = COMBINE ? U1 : K;
   const int u = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // this wave's unit
   const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x / (H / R);
-  const int h0 = (blockIdx.x - t * (H / R)) * R;
+  // (constant H: tokens x row blocks in x; else row blocks in x, tokens in y)
+  constexpr int kBlocks = H_ ? H_ / R : 1;
+  const int t = H_ ? blockIdx.x / kBlocks : blockIdx.y;
+  const int h0 = (H_ ? blockIdx.x % kBlocks : blockIdx.x) * R;
   const int r = lane / LPR;
   const int ch = lane & (LPR - 1);
   __shared__ float s_y[NU][R];
@@ -2093,7 +2124,8 @@ hipError_t launch_router_mfma(const DecodeArgs& a, float* wnorm, uint16_t* split
 
 hipError_t launch_rmsnorm(const uint16_t* x, const uint16_t* w, int T, int H, float eps,
                           uint16_t* out, hipStream_t s) {
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3((T + 3) / 4), dim3(256), 0, s, x, w, T, H, eps, out);
+  const auto k = H <= 2048 ? rmsnorm_kernel<4> : H <= 4096 ? rmsnorm_kernel<8> : rmsnorm_kernel<0>;
+  hipLaunchKernelGGL(k, dim3((T + 3) / 4), dim3(256), 0, s, x, w, T, H, eps, out);
   RMOE_CHECK_LAUNCH();
   return hipSuccess;
 }
@@ -2197,23 +2229,28 @@ hipError_t launch_down(const DecodeArgs& a, int bits, bool combine, hipStream_t 
   if (a.few_bits != 0 || a.act16) {
     // rows per workgroup: 16 up to 4 tokens, 8 beyond (16 where a pass of
     // the wave is that many)
-    auto go = [&](auto bits_c, auto combine_c, auto i_c) {
+    auto go = [&](auto bits_c, auto combine_c, auto h_c, auto i_c) {
       constexpr int B = decltype(bits_c)::value;
       constexpr bool C = decltype(combine_c)::value;
+      constexpr int HC = decltype(h_c)::value;
       constexpr int I = decltype(i_c)::value;
       constexpr int RS = B == 4 && I == 128 ? 16 : 8;
       const dim3 block(64 * kMaxFusedUnits);
+      const int nb = a.H / (a.T <= 4 ? 16 : RS);
+      const dim3 grid = HC ? dim3(nb * a.T) : dim3(nb, a.T);
       if (a.T <= 4)
-        hipLaunchKernelGGL((down_few_kernel<B, C, I, 16>), dim3((unsigned)(a.T * (a.H / 16))),
-                           block, 0, s, a);
+        hipLaunchKernelGGL((down_few_kernel<B, C, HC, I, 16>), grid, block, 0, s, a);
       else
-        hipLaunchKernelGGL((down_few_kernel<B, C, I, RS>), dim3((unsigned)(a.T * (a.H / RS))),
-                           block, 0, s, a);
+        hipLaunchKernelGGL((down_few_kernel<B, C, HC, I, RS>), grid, block, 0, s, a);
     };
     auto width = [&](auto bits_c, auto combine_c) {
-      if (a.I == 512) go(bits_c, combine_c, std::integral_constant<int, 512>{});
-      else if (a.I == 256) go(bits_c, combine_c, std::integral_constant<int, 256>{});
-      else go(bits_c, combine_c, std::integral_constant<int, 128>{});
+      using Any = std::integral_constant<int, 0>;
+      using Own = std::integral_constant<int, few::H>;
+      if (a.I == 512 && a.H == few::H)
+        go(bits_c, combine_c, Own{}, std::integral_constant<int, 512>{});
+      else if (a.I == 512) go(bits_c, combine_c, Any{}, std::integral_constant<int, 512>{});
+      else if (a.I == 256) go(bits_c, combine_c, Any{}, std::integral_constant<int, 256>{});
+      else go(bits_c, combine_c, Any{}, std::integral_constant<int, 128>{});
     };
     using B8 = std::integral_constant<int, 8>;
     using B4 = std::integral_constant<int, 4>;
@@ -2276,6 +2313,8 @@ static hipError_t qmv_cpl(const QmvArgs& a, hipStream_t s) {
 static bool qmv_rows_ok(const QmvArgs& a, int bits) {
   if (a.K % 256 || a.K > 4096 || (((uintptr_t)a.w.s | (uintptr_t)a.w.b) & 7)) return false;
   if (!a.lhs && !a.rhs) return a.M >= 32;
+  // (a launch holds fewer than 2^32 threads, up to 1024 per 64 columns here)
+  if ((long long)a.M * ((a.N + 63) / 64) >= 1ll << 22) return false;
   const bool many = a.M >= 128 || (a.M >= 64 && a.K <= (bits == 4 ? 2048 : 1024));
   return many && (long long)a.M * a.N * a.K >= 1ll << 25;
 }

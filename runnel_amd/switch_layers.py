@@ -180,9 +180,10 @@ class QuantizedSwitchLinear(_Params):
     def _gather(self, x, indices, lhs):
         """The product for x rows `lhs` (as _x_rows gives them)."""
         idx_shape = indices.shape
-        y = native.gather_qmm(x.reshape(-1, x.shape[-1]), self.weight, self.scales, self.biases,
-                              self.bits, self.group_size,
-                              rhs_indices=indices.reshape(-1), lhs_indices=lhs)
+        # (refuses x with more than one row per leading index)
+        x2 = x.reshape(x.shape[:-2].numel(), x.shape[-1])
+        y = native.gather_qmm(x2, self.weight, self.scales, self.biases, self.bits,
+                              self.group_size, rhs_indices=indices.reshape(-1), lhs_indices=lhs)
         if "bias" in self:
             y = y + self["bias"][indices.reshape(-1).long()]
         return y.reshape(*idx_shape, 1, self.output_dims)

@@ -566,3 +566,16 @@ def test_combine_and_swiglu_reject_before_launch():
     assert lib.rmoe_swiglu(FAKE, FAKE, -1, FAKE, None) == _lib.RMOE_EINVAL
     assert lib.rmoe_swiglu(FAKE, FAKE + 2, 8, FAKE, None) == _lib.RMOE_EALIGN
     assert lib.rmoe_swiglu(None, None, 0, None, None) == ok
+
+
+@pytest.mark.parametrize("shape", [(1, 2, 64), (5, 1, 2, 64), (5, 3, 2, 64)])
+def test_switch_linear_refuses_more_than_one_row_per_index(monkeypatch, shape):
+    """x is [..., 1 or k, 1, in]: with several rows where the 1 stands, the
+    row an index takes is not defined, and the call is refused before the
+    product."""
+    from runnel_amd import native
+    from runnel_amd.switch_layers import QuantizedSwitchLinear
+    monkeypatch.setattr(native, "gather_qmm", lambda *a, **k: pytest.fail("not refused"))
+    lin = QuantizedSwitchLinear(64, 8, 4)
+    with pytest.raises(RuntimeError, match="invalid for input"):
+        lin(torch.zeros(shape, dtype=torch.bfloat16), torch.zeros((5, 3), dtype=torch.int32))

@@ -252,9 +252,12 @@ class SparseMoeBlock(nn.Module):
         if self.shared_expert is not None:
             sh, sg = self.shared_expert(x2), self.shared_expert_gate(x2)
         res = None if residual is None else residual.reshape(-1, D)
-        rows = [t for t in (y, sh, res) if t is not None]
-        if (native.rows_ready(*rows) and y.dim() == 3 and D % 8 == 0
-                and (sg is None or (sg.dtype == BF16 and tuple(sg.shape) == (len(x2), 1)
+        T = len(x2)
+        tail = [t for t in (sh, res) if t is not None]
+        # (rows that broadcast, as a residual [1, D], take the torch form)
+        if (native.rows_ready(y, *tail) and tuple(y.shape) == (T, scores.shape[1], D)
+                and all(tuple(t.shape) == (T, D) for t in tail) and D % 8 == 0
+                and (sg is None or (sg.dtype == BF16 and tuple(sg.shape) == (T, 1)
                                     and not sg.requires_grad))):
             return native.combine(y, scores, sh, sg, res).reshape(*lead, D)
         out = (y.float() * scores[..., None]).sum(dim=-2)

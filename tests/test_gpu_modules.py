@@ -56,6 +56,16 @@ def _block_from_oracle(L, bits):
     return blk
 
 
+class _Call:
+    """A caller's own module in the block's place."""
+
+    def __init__(self, fn):
+        self.fn = fn
+
+    def __call__(self, *args):
+        return self.fn(*args)
+
+
 def _contract_mismatches(got_bits, ref_bits):
     g = M.bf16_to_f32(got_bits).astype(np.float64)
     r = M.bf16_to_f32(ref_bits).astype(np.float64)
@@ -127,3 +137,32 @@ def test_packed_module_call_per_slot(torch_cuda, bits):
         mode = "prefill" if T * 4 >= 64 else "contract"
         ref = M.f32_to_bf16(M.switch_glu(L, x, idx, mode).reshape(T * 4, 512))
         assert _contract_mismatches(got, ref) <= got.size // 500, T
+
+
+@pytest.mark.parametrize("what", ["residual", "shared", "slots"])
+def test_composed_block_broadcasts_rows(torch_cuda, what):
+    """Before packing, one residual row, one shared-expert row or one slot's
+    row may stand for all of them, as in the torch expression of the block:
+    bf16(residual + bf16(sum_j score_j y_j + sigmoid(g) shared)).  An fp32 sum
+    in another order may move each of the two roundings by one bf16 step
+    (2^-8 of its value)."""
+    torch = torch_cuda
+    from runnel_amd import native
+    L = M.make_layer(9300, hidden=512, inter=128, experts=32, top_k=4)
+    blk = _block_from_oracle(L, 8)
+    x = dev_bf16(M.make_x(9301, 6, 512))
+    res = dev_bf16(M.make_x(9302, 1, 512))
+    sm, se = blk.switch_mlp, blk.shared_expert
+    if what == "shared":
+        blk._modules["shared_expert"] = _Call(lambda v: se(v[:1]))
+    if what == "slots":
+        blk._modules["switch_mlp"] = _Call(lambda v, i: sm(v, i)[:, :1].contiguous())
+    inds, scores = native.router(blk.gate.weight, x, 4)
+    y = blk.switch_mlp(x, inds)
+    out = (y.double() * scores.double()[..., None]).sum(-2)
+    out = out + torch.sigmoid(blk.shared_expert_gate(x).double()) * blk.shared_expert(x).double()
+    ref = res.double() + out
+    got = blk(x, residual=res if what == "residual" else res.expand(6, 512).contiguous())
+    assert tuple(got.shape) == (6, 512)
+    tol = 2.0 ** -8 * (out.abs() + ref.abs()) * 1.01 + 1e-6
+    assert ((got.double() - ref).abs() <= tol).all()

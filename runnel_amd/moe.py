@@ -257,8 +257,7 @@ class SparseMoeBlock(nn.Module):
         # (rows that broadcast, as a residual [1, D], take the torch form)
         if (native.rows_ready(y, *tail) and tuple(y.shape) == (T, scores.shape[1], D)
                 and all(tuple(t.shape) == (T, D) for t in tail) and D % 8 == 0
-                and (sg is None or (sg.dtype == BF16 and tuple(sg.shape) == (T, 1)
-                                    and not sg.requires_grad))):
+                and (sg is None or (tuple(sg.shape) == (T, 1) and native.rows_ready(sg)))):
             return native.combine(y, scores, sh, sg, res).reshape(*lead, D)
         out = (y.float() * scores[..., None]).sum(dim=-2)
         if sh is not None:

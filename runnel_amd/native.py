@@ -12,6 +12,8 @@ import ctypes
 from dataclasses import dataclass
 
 import torch
+from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 from . import _lib
 
@@ -563,11 +565,28 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.
     return out.reshape(x.shape)
 
 
+def _plain_call() -> bool:
+    """Whether nothing else has to see an operation's torch form: no
+    forward-mode level, function transform (vmap, jvp, ...), dispatch or
+    function mode (a default device aside), trace or compilation is active."""
+    if (forward_ad._current_level >= 0 or torch.compiler.is_compiling()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() or torch._C._get_tracing_state() is not None):
+        return False
+    return all(isinstance(torch._C._get_function_stack_at(i), DeviceContext)
+               for i in range(torch._C._len_torch_function_stack()))
+
+
 def rows_ready(*tensors) -> bool:
-    """Whether every tensor is a contiguous, 16-byte aligned bf16 GPU tensor
-    outside autograd: what the row kernels below take as it is."""
-    return all(t.dtype == BF16 and t.is_cuda and t.is_contiguous() and not t.requires_grad
-               and t.data_ptr() % 16 == 0 for t in tensors)
+    """Whether the row kernels below may stand for the torch form of a call:
+    every tensor a plain, contiguous, 16-byte aligned bf16 tensor of the
+    current GPU outside autograd, and nothing that traces, transforms or
+    intercepts torch operations active."""
+    return (all(type(t) is torch.Tensor and t.dtype == BF16 and t.is_cuda and t.is_contiguous()
+                and not t.requires_grad for t in tensors)
+            and _plain_call()
+            and all(t.get_device() == torch.cuda.current_device() and t.data_ptr() % 16 == 0
+                    for t in tensors))
 
 
 def combine(y: torch.Tensor, weights: torch.Tensor, shared: torch.Tensor | None = None,
@@ -600,6 +619,9 @@ def combine(y: torch.Tensor, weights: torch.Tensor, shared: torch.Tensor | None 
                                 _lib.ptr(gate), _lib.ptr(residual), out.data_ptr(),
                                 _lib.stream_handle(y.device)))
     return out
+
+
+SWIGLU_MAX = 2048 * 0x7FFFFFFF // 256  # values of one rmoe_swiglu call
 
 
 def swiglu(up: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:

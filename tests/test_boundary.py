@@ -579,3 +579,43 @@ def test_switch_linear_refuses_more_than_one_row_per_index(monkeypatch, shape):
     lin = QuantizedSwitchLinear(64, 8, 4)
     with pytest.raises(RuntimeError, match="invalid for input"):
         lin(torch.zeros(shape, dtype=torch.bfloat16), torch.zeros((5, 3), dtype=torch.int32))
+
+
+def test_row_kernels_give_way_to_torch_transforms():
+    """The row kernels stand for a torch expression only where nothing else
+    has to see it."""
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from runnel_amd import native
+    seen = []
+
+    def note(x):
+        seen.append(native._plain_call())
+        return x * 1
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, fn, types, args=(), kwargs=None):
+            return fn(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, fn, types, args=(), kwargs=None):
+            return fn(*args, **(kwargs or {}))
+
+    x = torch.ones(2)
+    assert native._plain_call()
+    with torch.device("cpu"):
+        assert native._plain_call()
+    with forward_ad.dual_level():
+        note(x)
+    torch.vmap(note)(x)
+    torch.func.jvp(note, (x,), (x,))
+    torch.func.grad(lambda v: note(v).sum())(x)
+    with Function():
+        note(x)
+    with Dispatch():
+        note(x)
+    torch.jit.trace(note, x, check_trace=False)
+    assert seen == [False] * 7
+    assert not native.rows_ready(x.bfloat16())  # a host tensor

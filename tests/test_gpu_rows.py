@@ -66,3 +66,19 @@ def test_swiglu(torch_cuda, n):
     assert (ok | (got == ref) | (np.isnan(got) & np.isnan(ref))).all()
     fin = np.isfinite(ref)
     assert (got[fin] == ref[fin]).mean() >= 0.99 or n < 100
+
+
+def test_block_tail_under_forward_mode(torch_cuda):
+    """A residual's forward-mode tangent passes through the block before
+    packing (its other operands carry none)."""
+    torch = torch_cuda
+    from torch.autograd import forward_ad
+
+    from runnel_amd import SparseMoeBlock
+    blk = SparseMoeBlock(64, 64, 4, 2, shared_expert_intermediate_size=64, device="cuda")
+    x, r, t = torch.randn(3, 5, 64, device="cuda").bfloat16()
+    plain = blk(x, residual=r)
+    with forward_ad.dual_level():
+        out = forward_ad.unpack_dual(blk(x, residual=forward_ad.make_dual(r, t)))
+        assert torch.equal(out.primal, plain)  # (zero weights: the residual itself)
+        assert torch.equal(out.tangent, t)

@@ -189,16 +189,16 @@ class QuantizedSwitchLinear(_Params):
         return y.reshape(*idx_shape, 1, self.output_dims)
 
 
+# (a subclass's or a wrapper's own call is made, and not passed by)
+_SWITCH_LINEAR_CALL = QuantizedSwitchLinear.__call__
+
+
 def swiglu(x: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
-    return torch.nn.functional.silu(gate) * x
-
-
-def _activate(activation, x, gate):
-    """activation(x, gate); the package's own SwiGLU of two kernel outputs in
-    one launch."""
-    if type(activation) is SwiGLU and x.shape == gate.shape and native.rows_ready(x, gate):
+    """silu(gate) * x; two plain bf16 GPU tensors of one shape in one launch,
+    with the bits of the torch form."""
+    if native.rows_ready(x, gate) and x.shape == gate.shape and x.numel() <= native.SWIGLU_MAX:
         return native.swiglu(x, gate)
-    return activation(x, gate)
+    return torch.nn.functional.silu(gate) * x
 
 
 class SwiGLU(nn.Module):
@@ -207,9 +207,6 @@ class SwiGLU(nn.Module):
 
     def __call__(self, x, gate):
         return swiglu(x, gate)
-
-
-_SWIGLU = SwiGLU()
 
 
 class SwitchGLU(nn.Module):
@@ -231,12 +228,13 @@ class SwitchGLU(nn.Module):
     def __call__(self, x, indices):
         x = x.unsqueeze(-2).unsqueeze(-3)  # expand_dims(x, (-2, -3))
         up, gate = self.up_proj, self.gate_proj
-        if all(type(p) is QuantizedSwitchLinear and p.mode == "affine" for p in (up, gate)):
+        if all(type(p).__call__ is _SWITCH_LINEAR_CALL and p.mode == "affine"
+               for p in (up, gate)):
             lhs = _x_rows(x, indices)  # once for both
             x_up, x_gate = up._gather(x, indices, lhs), gate._gather(x, indices, lhs)
         else:
             x_up, x_gate = up(x, indices), gate(x, indices)
-        x = self.down_proj(_activate(self.activation, x_up, x_gate), indices)
+        x = self.down_proj(self.activation(x_up, x_gate), indices)
         return x.squeeze(-2)
 
 
@@ -251,4 +249,4 @@ class MLP(nn.Module):
         self.down_proj = QuantizedLinear(hidden_dim, dim, bits, group_size, device=device)
 
     def __call__(self, x):
-        return self.down_proj(_activate(_SWIGLU, self.up_proj(x), self.gate_proj(x)))
+        return self.down_proj(swiglu(self.up_proj(x), self.gate_proj(x)))

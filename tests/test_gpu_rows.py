@@ -68,6 +68,72 @@ def test_swiglu(torch_cuda, n):
     assert (got[fin] == ref[fin]).mean() >= 0.99 or n < 100
 
 
+def test_swiglu_function_keeps_the_torch_bits(torch_cuda):
+    """Every bf16 gate against up values of every kind: the kernel behind
+    switch_layers.swiglu gives the bits of silu(gate) * up (NaN for NaN)."""
+    torch = torch_cuda
+    from runnel_amd import native
+    from runnel_amd.switch_layers import swiglu
+    gate = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).cuda()
+    for u in (1.0, -0.7109375, 3.0e38, 1.0e-38, 0.0, -0.0, float("inf"), float("nan")):
+        up = torch.full_like(gate, u)
+        assert native.rows_ready(up, gate)
+        got, ref = swiglu(up, gate), torch.nn.functional.silu(gate) * up
+        same = (got.view(torch.int16) == ref.view(torch.int16)) | (got.isnan() & ref.isnan())
+        assert same.all(), u
+
+
+def test_swiglu_torch_form(torch_cuda):
+    """Rows the kernel does not take: in autograd, not contiguous, not 16-byte
+    aligned, of broadcasting shapes, with a forward-mode tangent."""
+    torch = torch_cuda
+    from torch.autograd import forward_ad
+
+    from runnel_amd import native
+    from runnel_amd.switch_layers import swiglu
+    up, gate = torch.randn(2, 48, 64, device="cuda").bfloat16()
+    form = lambda u, g: torch.nn.functional.silu(g) * u
+    pad = torch.randn(2, 48 * 64 + 8, device="cuda").bfloat16()
+    for u, g in ((up.t(), gate.t()), (pad[0, 1:3073], pad[1, 1:3073]), (up, gate[:1])):
+        assert not native.rows_ready(u, g) or u.shape != g.shape
+        assert torch.equal(swiglu(u, g), form(u, g))
+    u, g = up.clone().requires_grad_(), gate.clone().requires_grad_()
+    swiglu(u, g).sum().backward()
+    u2, g2 = up.clone().requires_grad_(), gate.clone().requires_grad_()
+    form(u2, g2).sum().backward()
+    assert torch.equal(u.grad, u2.grad) and torch.equal(g.grad, g2.grad)
+    with forward_ad.dual_level():
+        out = swiglu(forward_ad.make_dual(up, gate), forward_ad.make_dual(gate, up))
+        ref = form(forward_ad.make_dual(up, gate), forward_ad.make_dual(gate, up))
+        assert torch.equal(forward_ad.unpack_dual(out).tangent,
+                           forward_ad.unpack_dual(ref).tangent)
+
+
+def test_replaced_calls_are_made(torch_cuda, monkeypatch):
+    """A program that wraps QuantizedSwitchLinear or SwiGLU sees every one of
+    their calls inside SwitchGLU, with the result unchanged."""
+    torch = torch_cuda
+    from runnel_amd import QuantizedSwitchLinear, SwiGLU, SwitchGLU
+    sm = SwitchGLU(64, 128, 4, device="cuda")
+    for p in (sm.gate_proj, sm.up_proj, sm.down_proj):
+        w = torch.randn(4, p.output_dims, p.input_dims, device="cuda") * 0.1
+        q = QuantizedSwitchLinear.from_float(w)
+        p.weight, p.scales, p.biases = q.weight, q.scales, q.biases
+    x = torch.randn(5, 64, device="cuda").bfloat16()
+    idx = torch.randint(0, 4, (5, 2), device="cuda", dtype=torch.int32)
+    ref = sm(x, idx)
+    calls = []
+    for cls in (QuantizedSwitchLinear, SwiGLU):
+        own = cls.__call__
+
+        def wrapped(self, *args, _own=own, _name=cls.__name__):
+            calls.append(_name)
+            return _own(self, *args)
+        monkeypatch.setattr(cls, "__call__", wrapped)
+    assert torch.equal(sm(x, idx), ref)
+    assert sorted(calls) == ["QuantizedSwitchLinear"] * 3 + ["SwiGLU"]
+
+
 def test_block_tail_under_forward_mode(torch_cuda):
     """A residual's forward-mode tangent passes through the block before
     packing (its other operands carry none)."""

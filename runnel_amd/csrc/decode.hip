@@ -2285,18 +2285,43 @@ hipError_t launch_down(const DecodeArgs& a, int bits, bool combine, hipStream_t 
   return hipSuccess;
 }
 
+// A launch holds fewer than 2^32 threads: calls of more rows go in pieces
+// (whole windows of qmv_rows_kernel where a piece holds one).
+// group_threads: the threads of `group` rows.
+template <typename F>
+static hipError_t qmv_pieces(const QmvArgs& a, long long group_threads, int group, F&& launch) {
+  long long n = 0xFFFFFFFFll / group_threads * group;
+  if (n < 1) return hipErrorInvalidValue;
+  if (n > kQmvWindow) n -= n % kQmvWindow;
+  for (long long m0 = 0; m0 < a.M; m0 += n) {
+    QmvArgs p = a;
+    p.M = (int)(a.M - m0 < n ? a.M - m0 : n);
+    if (a.lhs) {
+      p.lhs += m0;
+    } else {
+      p.x += m0 * a.K;
+      p.x_rows = p.M;
+    }
+    if (a.rhs) p.rhs += m0;
+    if (a.y_f32) p.y_f32 += m0 * a.N;
+    if (a.y_bf16) p.y_bf16 += m0 * a.N;
+    launch(p);
+    RMOE_CHECK_LAUNCH();
+  }
+  return hipSuccess;
+}
+
 template <int BITS, int CPL>
 static hipError_t qmv_cpl(const QmvArgs& a, hipStream_t s) {
   const int vpc = BITS == 8 ? 16 : 32;
   const int ch = a.K / vpc;
   const int lpr = ch >= 64 ? 64 : ch;
   const int rows_per_block = 4 * (64 / lpr);
-  const int bpr = (a.N + rows_per_block - 1) / rows_per_block;
-  const long long blocks = (long long)bpr * a.M;
-  hipLaunchKernelGGL((qmv_kernel<BITS, CPL>), dim3((unsigned)blocks), dim3(256),
-                     0, s, a, bpr);
-  RMOE_CHECK_LAUNCH();
-  return hipSuccess;
+  const int bpr = (int)(((long long)a.N + rows_per_block - 1) / rows_per_block);
+  return qmv_pieces(a, bpr * 256ll, 1, [&](const QmvArgs& p) {
+    hipLaunchKernelGGL((qmv_kernel<BITS, CPL>), dim3((unsigned)((long long)bpr * p.M)),
+                       dim3(256), 0, s, p, bpr);
+  });
 }
 
 // When a call takes qmv_rows_kernel (its slices are 256 values, up to
@@ -2313,8 +2338,6 @@ static hipError_t qmv_cpl(const QmvArgs& a, hipStream_t s) {
 static bool qmv_rows_ok(const QmvArgs& a, int bits) {
   if (a.K % 256 || a.K > 4096 || (((uintptr_t)a.w.s | (uintptr_t)a.w.b) & 7)) return false;
   if (!a.lhs && !a.rhs) return a.M >= 32;
-  // (a launch holds fewer than 2^32 threads, up to 1024 per 64 columns here)
-  if ((long long)a.M * ((a.N + 63) / 64) >= 1ll << 22) return false;
   const bool many = a.M >= 128 || (a.M >= 64 && a.K <= (bits == 4 ? 2048 : 1024));
   return many && (long long)a.M * a.N * a.K >= 1ll << 25;
 }
@@ -2324,13 +2347,15 @@ static hipError_t qmv_rows(const QmvArgs& a, hipStream_t s) {
   const int ks = a.K / QmvRows<BITS, NB>::L;
   const int cg = ks <= 4 ? 4 / ks : 1;
   const int per = 16 * NB * cg;
-  const int bpr = (a.N + per - 1) / per;
-  const long long groups = DENSE ? (a.M + 15) / 16 : a.M;
+  const int bpr = (int)(((long long)a.N + per - 1) / per);
+  const int threads = 64 * ks * cg;
+  constexpr int kGroup = DENSE ? 16 : 1;
   const size_t lds = ks > 1 ? (size_t)ks * cg * 2 * 64 * sizeof(f32x4_r) : 0;
-  hipLaunchKernelGGL((qmv_rows_kernel<BITS, NB, DENSE>), dim3((unsigned)(bpr * groups)),
-                     dim3(64 * ks * cg), lds, s, a, bpr, ks);
-  RMOE_CHECK_LAUNCH();
-  return hipSuccess;
+  return qmv_pieces(a, (long long)bpr * threads, kGroup, [&](const QmvArgs& p) {
+    const long long groups = (p.M + kGroup - 1) / kGroup;
+    hipLaunchKernelGGL((qmv_rows_kernel<BITS, NB, DENSE>), dim3((unsigned)(bpr * groups)),
+                       dim3(threads), lds, s, p, bpr, ks);
+  });
 }
 
 hipError_t launch_qmv(const QmvArgs& a, int bits, hipStream_t s) {

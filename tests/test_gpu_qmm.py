@@ -142,3 +142,44 @@ def test_rows_sharing_experts(torch_cuda, bits, Mr, N, K, E):
     err = np.abs(got - ref)
     assert (err <= K * 2.0 ** -24 * bound).all()
     assert np.linalg.norm(err) <= 4 * 2.0 ** -24 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("Mr,N,K,index", [
+    (131072 + 600, 2048, 4096, "both"),   # qmv_rows_kernel, 2^15 threads a row
+    (131072 + 600, 2048, 4096, "rhs"),    # and x in order
+    (262144 + 48, 4096, 4096, "none"),    # the same on one matrix, 16 rows a group
+    (262144 + 5, 2048, 128, "rhs"),       # qmv_kernel, 2^14 threads a row
+])
+def test_calls_of_more_than_one_launch(torch_cuda, Mr, N, K, index):
+    """Products of 2^32 threads and more (K and N chosen for the most threads
+    a row).  The rows repeat with a period of 4095, which divides no piece, so
+    every piece has to find its own x rows, indices and output rows; a row's
+    value does not depend on the others, so the repeats are equal bit for
+    bit."""
+    torch = torch_cuda
+    from runnel_amd import native
+    print(f"{Mr} x {N} x {K}, indices: {index}", flush=True)
+    P, E = 4095, 1 if index == "none" else 3
+    rng = np.random.default_rng(Mr + K)
+    w = rng.standard_normal((E, N, K), dtype=np.float32) * np.float32(0.02)
+    wq, s, b = native.quantize(torch.from_numpy(w).cuda(), 8)
+    base = dev_bf16(M.make_x(31, P, K))
+    at = torch.arange(Mr, device="cuda") % P
+    rhs = (at % E).to(torch.int32)
+    dt = torch.float32 if index == "none" else torch.bfloat16
+    if index == "none":
+        y = native.gather_qmm(base[at], wq[0], s[0], b[0], 8, out_dtype=dt)
+    elif index == "rhs":
+        y = native.gather_qmm(base[at], wq, s, b, 8, rhs_indices=rhs, out_dtype=dt)
+    else:
+        y = native.gather_qmm(base, wq, s, b, 8, rhs_indices=rhs,
+                              lhs_indices=at.to(torch.int32), out_dtype=dt)
+    torch.cuda.synchronize()
+    first = y[:P]
+    for r in range(P, Mr, P):
+        assert torch.equal(y[r:r + P], first[:Mr - r]), r
+    few = torch.arange(0, P, 97, device="cuda")
+    wf = native.dequantize(wq, s, b, 8).double()
+    ref = torch.stack([wf[int(rhs[i])] @ base[i].double() for i in few])
+    err = (first[few].double() - ref).norm() / ref.norm()
+    assert err <= (2.0 ** -8 if dt == torch.bfloat16 else 1e-6)

@@ -2325,21 +2325,39 @@ static hipError_t qmv_cpl(const QmvArgs& a, hipStream_t s) {
 }
 
 // When a call takes qmv_rows_kernel (its slices are 256 values, up to
-// sixteen, their group parameters words of 8 bytes), us against qmv_kernel,
-// experts of 512 x 2048 / 2048 x 512 / 512 x 4096 (N x K):
-//   gathered rows, 4 bits: 64 rows 16.9 -> 12.0, 16.8 -> 11.4, 25.4 -> 25.7;
-//     130: 29.6 -> 22.7, 28.7 -> 20.1, 44.2 -> 38.8; 320: 74.9 -> 45.2,
-//     71.9 -> 38.1, 124 -> 64
-//   8 bits: 96 rows 24.5 -> 25.8, 30.7 -> 21.7; 130: 29.9 -> 28.5, 38.5 ->
-//     24.4, 53.0 -> 49.6; 320: 84 -> 57, 103 -> 49, 148 -> 69
-//   small products lose (96 rows of 1024 x 256: 7.4 -> 7.8)
-//   one matrix, 40 rows: 10.9 -> 5.4, 10.4 -> 4.3, 16.2 -> 8.4; 16 rows of
-//     512 x 4096 at 8 bits lose (7.5 -> 9.0)
+// sixteen, their group parameters words of 8 bytes).  It takes 3.5 to 9 us
+// however small the call, longer with more slices; qmv_kernel's time grows
+// with M N K from 3 us.  Weights cold, us of qmv_kernel / qmv_rows_kernel:
+//   one matrix (N x K), 8 bits: 200 x 256 at 100 rows 3.8/4.0, at 256 5.4/4.0;
+//     512 x 512 at 31 rows 4.3/4.2, at 63 5.9/4.2; 64 x 1024 at 100 4.2/4.2;
+//     200 x 2048 at 40 5.6/5.8, at 63 7.5/6.0; 200 x 4096 at 40 8.4/9.5, at 48
+//     11.1/9.5; 2048 x 2048 at 32 26.4/6.2; a gate of one row x 2048 at 64
+//     3.1/4.8, x 1024 at 4096 4.8/4.0 (4 bits: lines within a tenth of these)
+//   gathered rows, experts of 512 x 2048 | 2048 x 512 (128 experts), 4 bits:
+//     64 rows 18/12 | 17/12, 128: 31/23 | 29/19, 512: 109/52 | 111/46; 8 bits:
+//     64 rows 19/16 | 21/15, 96: 26/27 | 30/23, 512: 122/62 | 162/54;
+//     1024 x 256 at 96 rows 10/10, at 128 12/10
+//   sixteen slices need rows that share an expert (a window of kQmvWindow rows
+//     holds kQmvWindow / experts of each): 512 x 4096, 8 bits, 128 rows of 4
+//     experts 45/23, of 128 61/67, 200 of 128 93/80, 320 of 256 152/131; 200 x
+//     4096, 512 of 256 experts 91/100
+//   narrow banks list the rows anew for few columns: 128 x 512 at 512 rows
+//     11/12 (4 experts), at 1024 19/14; 64 x 2048 at 320 10/11, at 1024 25/20;
+//     64 x 4096 at 512 21/24; one expert never pays: 64 x 2048 at 1024 26/31,
+//     200 x 4096 at 1024 110/159
 static bool qmv_rows_ok(const QmvArgs& a, int bits) {
   if (a.K % 256 || a.K > 4096 || (((uintptr_t)a.w.s | (uintptr_t)a.w.b) & 7)) return false;
-  if (!a.lhs && !a.rhs) return a.M >= 32;
-  const bool many = a.M >= 128 || (a.M >= 64 && a.K <= (bits == 4 ? 2048 : 1024));
-  return many && (long long)a.M * a.N * a.K >= 1ll << 25;
+  const long long mn = (long long)a.M * a.N, work = mn * a.K;
+  const int E = a.experts;
+  if (!a.lhs && !a.rhs)
+    return (a.M >= 32 && work >= 1ll << 23 && mn >= (a.K > 2048 ? 9600 : 8192)) ||
+           (a.M >= 4096 && a.K <= 1024);
+  if (a.M < 128 && (a.M < 64 || a.K > (bits == 4 ? 2048 : 1024))) return false;
+  if (E == 1 && a.N < 512 && (a.N < 192 || a.K > 1024)) return false;
+  if (a.K > 2048 && (4ll * a.M < 5ll * E || (a.N < 256 && (E > 128 || a.M < 4 * E)))) return false;
+  if (E == 1) return work >= 4ll << 24;
+  if (a.N >= 192) return work >= 2ll << 24;
+  return work >= (a.K > 2048 ? 12ll : a.K > 1024 && bits == 8 ? 5ll : 3ll) << 24;
 }
 
 template <int BITS, int NB, bool DENSE>

@@ -100,7 +100,10 @@ def test_dense_qmm_random_shapes(torch_cuda, bits, shape):
 @pytest.mark.parametrize("Mr,N,K,E", [
     (32, 80, 256, 1), (40, 512, 2048, 1), (63, 130, 3072, 1),      # one matrix
     (64, 2048, 512, 8), (130, 1100, 256, 3), (530, 144, 512, 40),  # gathered
-    (128, 520, 512, 1), (300, 64, 2048, 200), (128, 72, 4096, 5)])
+    (128, 520, 512, 1), (300, 64, 2048, 200), (128, 72, 4096, 5),
+    # either side of the lines below which qmv_kernel takes the call
+    (32, 1023, 256, 1), (32, 1025, 256, 1), (63, 153, 3072, 1), (63, 152, 3072, 1),
+    (1030, 72, 1024, 40), (1100, 64, 2048, 200), (128, 264, 4096, 5), (128, 264, 4096, 103)])
 def test_rows_sharing_experts(torch_cuda, bits, Mr, N, K, E):
     """Many rows a call, fp32 out: row groups that fill, exceed or just miss
     16, windows of 512 rows, column remainders, ids out of range (zero rows)

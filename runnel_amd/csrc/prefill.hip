@@ -1305,20 +1305,28 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillArgs 
 // --------------------------------------------------------------- launchers
 // 32-row tiles waste few MFMA rows and spread few rows per expert over many
 // workgroups; 128-row tiles share each dequantised weight fragment across
-// more rows and pay once their workgroups fill the device.  R = rows per
-// expert on average; whole block in us, 32- against 128-row tiles, 8 bits |
-// 4 bits:
-//   hidden 2048, 256 experts: R 24 243/253 | 182/185, 32 281/270 | 217/208,
-//     48 351/293 | 272/239
-//   4096, 64 experts: R 44 215/207 | 161/166, 52 231/218 | 172/177,
-//     72 286/234 | 216/208
-//   1024, 128 experts: R 48 85/85 | 75/81, 64 94/91 | 85/88, 96 111/103 | 99/101
-//   512, 32 experts: R 72 43/56 | 41/55, 128 57/67 | 55/67
-// so 128 rows from R = 30 on if a call has `enough` 32-row gate/up tiles.
+// more rows, but their workgroups must fill the device.  R = rows per expert
+// on average, W = the 128-row gate/up tiles they make (an expert's last tile
+// half full).  Whole block in us, 32- against 128-row tiles, 8 bits | 4 bits,
+// weights cold, hidden x intermediate x experts:
+//   R 30 to 48 pays from two workgroups per CU on (W 512): 2048 x 512 x 256
+//     at R 24 268/269 | 202/202, at 36 333/300 | 266/246; 3584 x 512 x 64 (W
+//     256) at R 36 175/183 | 144/157
+//   beyond, W sqrt(R) sets it, the line higher for small hidden sizes (a
+//     tile's fixed part) and for 4 bits (less weight to share): 2560 x 256 x
+//     60 at R 48 134/137 | 119/134, at 80 184/167 | 163/165, at 128 259/215 |
+//     233/212; 512 x 512 x 64 at R 64 69/71 | 62/70, at 128 96/86 | 88/85;
+//     2048 x 128 x 32 at R 128 93/103 | 86/102, at 384 203/179 | 181/176
+// Over 20 sizes x 13 values of R x both widths, blocks and switch calls, none
+// is over 5% slower than with one line at R 48 (calls without a shared expert
+// would take 128 rows from R 24 on: up to 1.25 times as fast there).
 int prefill_tile_rows(int T, int K, int E, int H, int I, int bits) {
-  const long rows = (long)T * K;
-  const long enough = bits == 4 && H <= 1024 ? 1500 : 800;  // (1024 x 4 bits: R 91)
-  return rows <= 30L * E || rows / 32 * (I / 64) <= enough ? 32 : kPrefillBM;
+  const float R = (float)T * K / E;
+  if (R <= 30.0f) return 32;
+  const float W = E * fmaxf(1.0f, R / 128 + 0.5f) * (I / 128);
+  if (R <= 48.0f) return W >= 512 ? kPrefillBM : 32;
+  const float line = (850.0f + 600.0f * 1024 / H) * (bits == 4 ? 1.3f : 1.0f);
+  return W * sqrtf(R) >= line ? kPrefillBM : 32;
 }
 
 int prefill_sort_slices(int T, int K) {

@@ -259,11 +259,12 @@ def test_long_prefill_skewed_routing_4bit(torch_cuda):
     assert cosine(got.reshape(-1), mx_.reshape(-1)) >= MIN_COS
 
 
-@pytest.mark.parametrize("bits,T", [(8, 800), (8, 808), (4, 1496), (4, 1504)])
+@pytest.mark.parametrize("bits,T", [(8, 800), (8, 808), (8, 1022), (8, 1023), (4, 1496),
+                                    (4, 1504), (4, 1233), (4, 1234)])
 def test_tile_height_rule(torch_cuda, bits, T):
-    """Either side of the work at which a call takes 128-row tiles (800
-    32-row gate/up tiles, 1500 at 4 bits and hidden up to 1024; 8 experts of
-    intermediate 512, so rows per expert are far past the other condition)."""
+    """Calls of a few experts with hundreds of rows each, on both sides of
+    the line (1023 and 1234 tokens here) from which a call takes
+    128-row tiles."""
     L = M.make_layer(77 + bits, hidden=256, inter=512, experts=8, top_k=4, bits=bits,
                      shared=False)
     x = M.make_x(7 + T, T, 256)

@@ -746,7 +746,7 @@ int block_launch(const rmoe_layer* L, const uint16_t* x, int32_t tokens,
   a.scores_out = scores_out;
   if (few_eligible(L, tokens, lay.rows != 0)) a.few_bits = L->gate_up.bits;
   a.logit_planes = lay.rows ? rmoe::router_logit_planes(tokens) : 1;
-  if (lay.rows && tokens > rmoe::router_direct_tokens(router_quantized(L)) &&
+  if (lay.rows && !rmoe::router_direct(tokens, L->experts, L->hidden, router_quantized(L)) &&
       rmoe::router_mfma_eligible(L->experts, L->hidden))
     e = rmoe::launch_router_mfma(
         a, reinterpret_cast<float*>(static_cast<char*>(ws) + lay.wnorm),

@@ -2045,18 +2045,24 @@ bool router_mfma_eligible(int E, int H) {
   return E % 64 == 0 && E <= 256 && H % 512 == 0 && H <= 4096;
 }
 
-// Tokens up to which the exact router in one launch beats logits and
-// selection (two launches, three with an 8-bit gate, whose weights are split;
-// its columns below are from when each plane took a launch of its own):
-// whole block in us, matrix-core router against router_kernel, 4 bits, at
-// hidden 2048 | 1024 | 4096 (256 | 128 | 64 experts).
-//   8-bit gate: 16 tokens 88.8 -> 66.8 | 49.4 -> 37.5 | 92.5 -> 70.6;
-//     48: 131.2 -> 127.2 | 54.0 -> 44.2 | 103.1 -> 81.3; 96: 150.0 -> 148.8 |
-//     57.8 -> 52.0 | 117.7 -> 97.4; 192: 162.0 -> 178.3 | 61.6 -> 63.4 | ..
-//   bf16 gate: 16 tokens 79.3 -> 76.2 | 42.5 -> 36.8 | 76.3 -> 70.3;
-//     24: 96.1 -> 94.8 | 44.7 -> 40.5 | 83.7 -> 77.6; 32: 102.9 -> 110.4 |
-//     45.3 -> 42.0 | 85.5 -> 79.8; 64: 129.4 -> 138.8 | 45.9 -> 52.2 | ..
-int router_direct_tokens(bool rq8) { return rq8 ? 96 : 24; }
+// Whether the exact router in one launch beats logits and selection (two
+// launches; three with an 8-bit gate, whose weights are split).  Its vector
+// work grows with tokens x experts (hidden sizes differ little), which sets
+// the line.  Whole block in us, matrix-core router against router_kernel, 4
+// bits, weights cold, hidden 2048 x 256 experts | 1024 x 128 | 2048 x 64:
+//   bf16 gate: 24 tokens 92.2/90.8 | 47.5/43.1 | 65.6/59.2; 28: 98.7/97.4 |
+//     47.8/44.0 | 64.7/58.4; 32: 106.2/106.9 | 48.2/44.9 | 67.9/61.5; 56: ..
+//     | 48.8/48.2 | 71.9/67.3; 64: .. | 50.4/51.3 | 72.5/68.3; 112: .. | .. |
+//     76.8/72.7; 192: hidden 512 x 64 1 us faster, 4096 x 64 2.5 slower
+//   8-bit gate: 48 tokens 127.7/123.6 | 52.9/46.8 | 77.3/66.0; 56: 129.2/126.2
+//     | 52.6/47.9 | 77.9/67.8; 64: 130.9/131.2 | 54.7/51.7 | 78.4/68.9; 112: ..
+//     | 57.5/57.1 | 82.6/72.6; 128: .. | 59.4/61.0 | 83.5/76.9; 192: .. | .. |
+//     88.2/82.6; 256: .. | .. | 95.0/92.4.  Rows past 2048 take the selection's
+//     wide re-check: 4096 x 256 experts at 64 124.5/111.7, at 96 128.0/123.3,
+//     at 112 128.1/125.8; 4096 x 64 at 256 129.9/124.5, at 384 140.6/142.5
+bool router_direct(int T, int E, int H, bool rq8) {
+  return T * E <= (!rq8 ? 7168 : H > 2048 ? 24576 : 14336);
+}
 
 // 64 x 64 tiles (two workgroups of four waves per CU) from 4096 tokens on,
 // 32 x 32 below, where 64-token tiles leave most CUs idle: at 512 tokens

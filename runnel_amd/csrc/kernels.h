@@ -145,7 +145,7 @@ hipError_t launch_swiglu(const uint16_t* up, const uint16_t* gate, int64_t n, ui
                          hipStream_t s);
 // Many-token router on the matrix cores with exact selection (prefill).
 bool router_mfma_eligible(int E, int H);
-int router_direct_tokens(bool rq8);  // up to this many tokens launch_router is faster
+bool router_direct(int T, int E, int H, bool rq8);  // whether launch_router is faster
 int router_logit_planes(int T);
 // wnorm: [E] floats; split: [2, E, H] bf16 (quantized gates only)
 hipError_t launch_router_mfma(const DecodeArgs& a, float* wnorm, uint16_t* split,

@@ -11,11 +11,24 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // values each, so a load instruction reads whole lines; a wave takes 16
 // groups (each row of 16 lanes four neighbouring ones), all requested before
 // the first is used.  One thread per group read 16 bytes of 64 lines with
-// every load: 134 M values at 8 bits took 167 us (4.1 TB/s, in and out), now
-// 142 (4.8).
+// every load: 134 M values at 8 | 4 bits took 164 | 130 us (4.1 | 4.7 TB/s, in
+// and out), now 116 | 107 (5.9 | 5.7).
 // Arithmetic is plain IEEE fp32 (correctly rounded division, round-half-even
 // rint), so the result is reproducible on the host bit for bit.
 constexpr int kQuantGroups = 16;  // groups per wave
+
+// The value of lane u of each four.
+__device__ __forceinline__ float quad_bcast(float v, int u) {
+  const int i = __float_as_int(v);
+  int r;
+  switch (u) {  // the control must be a compile-time constant
+    case 0: r = __builtin_amdgcn_update_dpp(0, i, 0x00, 0xF, 0xF, false); break;
+    case 1: r = __builtin_amdgcn_update_dpp(0, i, 0x55, 0xF, 0xF, false); break;
+    case 2: r = __builtin_amdgcn_update_dpp(0, i, 0xAA, 0xF, 0xF, false); break;
+    default: r = __builtin_amdgcn_update_dpp(0, i, 0xFF, 0xF, 0xF, false); break;
+  }
+  return __int_as_float(r);
+}
 
 template <int BITS>
 __global__ __launch_bounds__(256) void quantize_kernel(const float* __restrict__ w,
@@ -35,11 +48,13 @@ __global__ __launch_bounds__(256) void quantize_kernel(const float* __restrict__
     v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(w + g * 64) + l16);
   }
   const float n_bins = (float)((1 << BITS) - 1);
-  uint32_t s_mine = 0, b_mine = 0;
+  // extremes of the groups: lane l16 keeps those of group l16 & 3 and works
+  // out that one's scale and bias (every lane those of all four, three
+  // divisions each, took 138 | 141 us)
+  const int mine = l16 & 3;
+  float w_max = 0.0f, w_min = 0.0f;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    // extremes of the group; a NaN only counts as its first value (the
-    // sequential "larger than" scan from value 0 that defines the format)
     float hi = fmaxf(fmaxf(v[u].x, v[u].y), fmaxf(v[u].z, v[u].w));
     float lo = fminf(fminf(v[u].x, v[u].y), fminf(v[u].z, v[u].w));
     hi = fmaxf(hi, dpp_f(hi, 0xB1));
@@ -50,35 +65,47 @@ __global__ __launch_bounds__(256) void quantize_kernel(const float* __restrict__
     lo = fminf(lo, dpp_f(lo, 0x141));
     hi = fmaxf(hi, dpp_f(hi, 0x140));
     lo = fminf(lo, dpp_f(lo, 0x140));
-    const float first = __shfl(v[u].x, lane & 48, 64);
-    const float w_max = first != first ? first : hi;
-    const float w_min = first != first ? first : lo;
-    const bool mask = fabsf(w_min) > fabsf(w_max);
-    float scale = (w_max - w_min) / n_bins;
-    scale = scale > 1e-7f ? scale : 1e-7f;
-    scale = mask ? scale : -scale;
-    const float edge = mask ? w_min : w_max;
-    const float q0 = rintf(edge / scale);
-    if (q0 != 0.0f) scale = edge / q0;
-    const float bias = q0 == 0.0f ? 0.0f : edge;
-    const uint32_t sb = f32_to_bf16(scale);
-    const uint32_t bb = f32_to_bf16(bias);
-    if (l16 == u) {
-      s_mine = sb;
-      b_mine = bb;
+    w_max = mine == u ? hi : w_max;
+    w_min = mine == u ? lo : w_min;
+  }
+  // a NaN only counts as its group's first value (the sequential "larger
+  // than" scan from value 0 that defines the format)
+  bool nan = false;
+#pragma unroll
+  for (int u = 0; u < U; ++u) nan = nan || v[u].x != v[u].x;
+  if (__any(nan && l16 == 0)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float first = __shfl(v[u].x, lane & 48, 64);
+      if (mine == u && first != first) w_max = w_min = first;
     }
-    const float s = bf16_to_f32(sb);
-    const float b = bf16_to_f32(bb);
-    // rint of the correctly rounded quotient.  The product with the rounded
-    // reciprocal is within 3 x 2^-24 |t| of that quotient: under 4.7e-5 for
-    // |t| < 260, and beyond that both clamp alike.  So unless t lies within
-    // 1e-4 of a half-integer (or is not finite, or the reciprocal is near the
-    // ends of its range) the two round to the same whole number; the others
-    // divide.  (A division per value took 162 us of vector work.)
-    const float r = 1.0f / s;
-    const bool plain = fabsf(s) > 0x1p-100f && fabsf(s) < 0x1p100f;
+  }
+  const bool mask = fabsf(w_min) > fabsf(w_max);
+  float scale = (w_max - w_min) / n_bins;
+  scale = scale > 1e-7f ? scale : 1e-7f;
+  scale = mask ? scale : -scale;
+  const float edge = mask ? w_min : w_max;
+  const float q0 = rintf(edge / scale);
+  if (q0 != 0.0f) scale = edge / q0;
+  const uint32_t sb = f32_to_bf16(scale);
+  const uint32_t bb = f32_to_bf16(q0 == 0.0f ? 0.0f : edge);
+  const float s_own = bf16_to_f32(sb);
+  const float b_own = bf16_to_f32(bb);
+  // Codes: rint of the correctly rounded quotient.  The product with the
+  // rounded reciprocal is within 3 x 2^-24 |t| of that quotient: under 4.7e-5
+  // for |t| < 260, and beyond that both clamp alike.  So unless t lies within
+  // 1e-4 of a half-integer (or is not finite, or the reciprocal is near the
+  // ends of its range: NaN here) the two round to the same whole number; the
+  // others divide.  (A division per value took 162 us at 8 bits.)
+  const bool plain = fabsf(s_own) > 0x1p-100f && fabsf(s_own) < 0x1p100f;
+  const float r_own = plain ? 1.0f / s_own : __builtin_nanf("");
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const float s = quad_bcast(s_own, u);
+    const float b = quad_bcast(b_own, u);
+    const float r = quad_bcast(r_own, u);
     float q4[4];
-    bool all = plain;
+    bool all = true;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float t = (v[u][j] - b) * r;
@@ -106,8 +133,8 @@ __global__ __launch_bounds__(256) void quantize_kernel(const float* __restrict__
     }
   }
   if (l16 < U && g0 + l16 < groups) {
-    s_out[g0 + l16] = (uint16_t)s_mine;
-    b_out[g0 + l16] = (uint16_t)b_mine;
+    s_out[g0 + l16] = (uint16_t)sb;
+    b_out[g0 + l16] = (uint16_t)bb;
   }
 }
 

@@ -1,5 +1,7 @@
 // Format kernels (affine quantize / dequantize) and the HBM stream
 // calibrator.
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -156,23 +158,21 @@ hipError_t launch_quantize(const float* w, int64_t rows, int cols, int bits,
 // fl32(q * s + b) with q * s exact, i.e. a single rounding, and optionally
 // bf16 (round-to-nearest-even) of it.  Bound by the output stream: a thread
 // writes 8 values per step in 16-byte pieces (V: the outputs are 16-byte
-// aligned) and has kDequantSteps steps' loads in flight.  Rows are whole
-// groups, so words, groups and outputs are all linear in the value index.
-// One packed word per thread with 2-byte stores took 136 us for 134 M values
-// at 8 bits to bf16 (3.0 TB/s, in and out), now 72 (5.7).
-constexpr int kDequantSteps = 4;
-
-template <int BITS, bool V>
+// aligned) and has STEPS steps' loads in flight.  Rows are whole groups, so
+// words, groups and outputs are all linear in the value index.
+// One packed word per thread with 2-byte stores took 138 us for 134 M values
+// at 8 bits to bf16 (3.0 TB/s, in and out), now 71 (5.8).
+template <int BITS, bool V, int STEPS>
 __global__ __launch_bounds__(256) void dequantize_kernel(const QW q, const int64_t value0,
                                                          const int64_t chunks,
                                                          float* __restrict__ out_f32,
                                                          uint16_t* __restrict__ out_bf16) {
   constexpr int WPC = BITS / 4;  // words per 8 values
-  const int64_t c0 = (int64_t)blockIdx.x * (256 * kDequantSteps) + threadIdx.x;
-  uint32_t word[kDequantSteps][WPC];
-  uint32_t sv[kDequantSteps], bv[kDequantSteps];
+  const int64_t c0 = (int64_t)blockIdx.x * (256 * STEPS) + threadIdx.x;
+  uint32_t word[STEPS][WPC];
+  uint32_t sv[STEPS], bv[STEPS];
 #pragma unroll
-  for (int k = 0; k < kDequantSteps; ++k) {
+  for (int k = 0; k < STEPS; ++k) {
     const int64_t c = c0 + 256 * k < chunks ? c0 + 256 * k : chunks - 1;
     const int64_t at = (value0 >> 3) + c;
     __builtin_memcpy(word[k], __builtin_assume_aligned(q.w + at * WPC, 4 * WPC), 4 * WPC);
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const QW q, const int64
     bv[k] = q.b[at >> 3];
   }
 #pragma unroll
-  for (int k = 0; k < kDequantSteps; ++k) {
+  for (int k = 0; k < STEPS; ++k) {
     const int64_t c = c0 + 256 * k;
     if (c >= chunks) return;
     const float s = bf16_to_f32(sv[k]);
@@ -222,17 +222,34 @@ hipError_t launch_dequantize(const QW& q, int cols, int bits, int64_t row_begin,
                              hipStream_t st) {
   const int64_t chunks = rows * (cols / 8);
   if (chunks == 0) return hipSuccess;
-  const unsigned blocks =
-      (unsigned)((chunks + 256 * kDequantSteps - 1) / (256 * kDequantSteps));
   const bool vec = (((uintptr_t)out_f32 | (uintptr_t)out_bf16) & 15) == 0;
+  // Four steps a thread for bf16 alone from 2^24 values on (134 M at 8 | 4
+  // bits: 77 | 79 us with one, 71 | 63 with four; 16 M, read once, 12.7 | 12.5
+  // and 12.7 | 11.6; also where one would not fit a launch).  Fewer values
+  // leave the device idle with four (65536 at 8 bits: 1.9 and 2.5), and
+  // fp32's wider stores want the threads (134 M at 8 bits: 121 and 165).
+  const bool four = (!out_f32 && chunks >= 1 << 21) || chunks >= 1ll << 31;
+  const int per = four ? 1024 : 256;
+  const unsigned blocks = (unsigned)((chunks + per - 1) / per);
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, st, q, row_begin * (int64_t)cols, chunks,
                        out_f32, out_bf16);
   };
-  if (bits == 8)
-    vec ? go(dequantize_kernel<8, true>) : go(dequantize_kernel<8, false>);
-  else
-    vec ? go(dequantize_kernel<4, true>) : go(dequantize_kernel<4, false>);
+  auto steps = [&](auto bits_c, auto vec_c) {
+    constexpr int B = decltype(bits_c)::value;
+    constexpr bool V = decltype(vec_c)::value;
+    if (four) go(dequantize_kernel<B, V, 4>);
+    else go(dequantize_kernel<B, V, 1>);
+  };
+  using B8 = std::integral_constant<int, 8>;
+  using B4 = std::integral_constant<int, 4>;
+  if (bits == 8) {
+    if (vec) steps(B8{}, std::true_type{});
+    else steps(B8{}, std::false_type{});
+  } else {
+    if (vec) steps(B4{}, std::true_type{});
+    else steps(B4{}, std::false_type{});
+  }
   return hipGetLastError();
 }
 

@@ -117,3 +117,30 @@ def test_nan_and_infinity(torch_cuda, bits):
         assert np.isnan(M.bf16_to_f32(s[g:g + 1]))[0]
         assert np.array_equal(M.bf16_to_f32(b[g:g + 1]), np.float32([edge]), equal_nan=True)
         assert not codes[g].any()
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("both", [False, True])
+def test_dequantize_from_the_longest_split_on(torch_cuda, bits, both):
+    """2^24 values and one group on either side: bf16 alone takes four steps a
+    thread from there on; with an fp32 output a thread takes one."""
+    torch = torch_cuda
+    from runnel_amd import _lib, native
+    for groups in (2 ** 18 - 1, 2 ** 18, 2 ** 18 + 1):
+        g = torch.Generator().manual_seed(groups + bits)
+        wq = torch.randint(-2 ** 31, 2 ** 31 - 1, (groups, 2 * bits), generator=g,
+                           dtype=torch.int32)
+        s, b = torch.randn((2, groups, 1), generator=g).bfloat16()
+        dev = (wq.cuda(), s.cuda(), b.cuda())
+        qw = native.qweight_struct(*dev, bits)
+        b16 = torch.empty((groups, 64), dtype=torch.bfloat16, device="cuda")
+        f32 = torch.empty((groups, 64), device="cuda") if both else None
+        _lib.check(_lib.load().rmoe_dequantize(ctypes.byref(qw), 0, groups, _lib.ptr(f32),
+                                               b16.data_ptr(), _lib.stream_handle(b16.device)))
+        q = wq.view(torch.uint8)
+        if bits == 4:
+            q = torch.stack((q & 15, q >> 4), -1).reshape(groups, 64)
+        # the product of a code and a bf16 scale fits fp32, so this rounds once
+        ref = (q.float() * s.float()).double() + b.double()
+        assert torch.equal(b16.cpu(), ref.float().bfloat16())
+        assert f32 is None or torch.equal(f32.cpu(), ref.float())

@@ -2241,7 +2241,7 @@ hipError_t launch_down(const DecodeArgs& a, int bits, bool combine, hipStream_t 
       constexpr int HC = decltype(h_c)::value;
       constexpr int I = decltype(i_c)::value;
       constexpr int RS = B == 4 && I == 128 ? 16 : 8;
-      const dim3 block(64 * kMaxFusedUnits);
+      const dim3 block(64 * (a.K + (C ? a.has_shared : 0)));  // a wave per unit
       const int nb = a.H / (a.T <= 4 ? 16 : RS);
       const dim3 grid = HC ? dim3(nb * a.T) : dim3(nb, a.T);
       if (a.T <= 4)

@@ -253,12 +253,13 @@ class SparseMoeBlock(nn.Module):
             sh, sg = self.shared_expert(x2), self.shared_expert_gate(x2)
         res = None if residual is None else residual.reshape(-1, D)
         T = len(x2)
-        tail = [t for t in (sh, res) if t is not None]
+        rows = [t for t in (sh, res) if t is not None]
+        gates = [] if sg is None else [sg]
         # (rows that broadcast, as a residual [1, D], take the torch form)
-        if (native.rows_ready(y, *tail) and tuple(y.shape) == (T, scores.shape[1], D)
-                and all(tuple(t.shape) == (T, D) for t in tail) and D % 8 == 0
-                and (sg is None or (tuple(sg.shape) == (T, 1) and native.rows_ready(sg)))):
-            return native.combine(y, scores, sh, sg, res).reshape(*lead, D)
+        if (native.rows_ready(y, *rows, *gates) and y.shape == (T, scores.shape[1], D)
+                and all(t.shape == (T, D) for t in rows) and D % 8 == 0
+                and (sg is None or sg.shape == (T, 1))):
+            return native._combine(y, scores, sh, sg, res).reshape(*lead, D)
         out = (y.float() * scores[..., None]).sum(dim=-2)
         if sh is not None:
             out = out + torch.sigmoid(sg.float()) * sh.float()

@@ -569,12 +569,13 @@ def _plain_call() -> bool:
     """Whether nothing else has to see an operation's torch form: no
     forward-mode level, function transform (vmap, jvp, ...), dispatch or
     function mode (a default device aside), trace or compilation is active."""
-    if (forward_ad._current_level >= 0 or torch.compiler.is_compiling()
-            or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch._C._len_torch_dispatch_stack() or torch._C._get_tracing_state() is not None):
+    if (forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() or torch.compiler.is_compiling()
+            or torch._C._get_tracing_state() is not None):
         return False
-    return all(isinstance(torch._C._get_function_stack_at(i), DeviceContext)
-               for i in range(torch._C._len_torch_function_stack()))
+    n = torch._C._len_torch_function_stack()
+    return n == 0 or all(isinstance(torch._C._get_function_stack_at(i), DeviceContext)
+                         for i in range(n))
 
 
 def rows_ready(*tensors) -> bool:
@@ -582,11 +583,16 @@ def rows_ready(*tensors) -> bool:
     every tensor a plain, contiguous, 16-byte aligned bf16 tensor of the
     current GPU outside autograd, and nothing that traces, transforms or
     intercepts torch operations active."""
-    return (all(type(t) is torch.Tensor and t.dtype == BF16 and t.is_cuda and t.is_contiguous()
-                and not t.requires_grad for t in tensors)
-            and _plain_call()
-            and all(t.get_device() == torch.cuda.current_device() and t.data_ptr() % 16 == 0
-                    for t in tensors))
+    for t in tensors:
+        if type(t) is not torch.Tensor or not t.is_cuda or t.dtype != BF16 or t.requires_grad:
+            return False
+    if not _plain_call():
+        return False
+    device = torch.cuda.current_device()
+    for t in tensors:
+        if t.get_device() != device or not t.is_contiguous() or t.data_ptr() % 16:
+            return False
+    return True
 
 
 def combine(y: torch.Tensor, weights: torch.Tensor, shared: torch.Tensor | None = None,
@@ -596,7 +602,6 @@ def combine(y: torch.Tensor, weights: torch.Tensor, shared: torch.Tensor | None 
     bf16 [T, k, H] (fp32 sums, slots in order), then + residual in bf16:
     weights float32 [T, k], shared bf16 [T, H] with gate logits bf16 [T] or
     both None -> bf16 [T, H]."""
-    lib = _lib.load()
     if y.dtype != BF16 or y.dim() != 3:
         raise ValueError("y must be a bfloat16 [tokens, k, hidden] tensor")
     T, k, H = y.shape
@@ -613,11 +618,16 @@ def combine(y: torch.Tensor, weights: torch.Tensor, shared: torch.Tensor | None 
         _check_rows(residual, "residual", T, H)
         residual = residual.contiguous()
     _require_cuda(y, weights, shared, gate, residual)
-    y, weights = y.contiguous(), weights.contiguous()
+    return _combine(y.contiguous(), weights.contiguous(), shared, gate, residual)
+
+
+def _combine(y, weights, shared, gate, residual):
+    """combine() of operands that need no check."""
+    T, k, H = y.shape
     out = torch.empty((T, H), dtype=BF16, device=y.device)
-    _lib.check(lib.rmoe_combine(y.data_ptr(), weights.data_ptr(), T, k, H, _lib.ptr(shared),
-                                _lib.ptr(gate), _lib.ptr(residual), out.data_ptr(),
-                                _lib.stream_handle(y.device)))
+    _lib.check(_lib.load().rmoe_combine(
+        y.data_ptr(), weights.data_ptr(), T, k, H, _lib.ptr(shared), _lib.ptr(gate),
+        _lib.ptr(residual), out.data_ptr(), _lib.stream_handle(y.device)))
     return out
 
 
@@ -626,14 +636,17 @@ SWIGLU_MAX = 2048 * 0x7FFFFFFF // 256  # values of one rmoe_swiglu call
 
 def swiglu(up: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     """bf16(bf16(silu(gate)) * up) of two bf16 tensors of one shape."""
-    lib = _lib.load()
     if up.dtype != BF16 or gate.dtype != BF16 or up.shape != gate.shape:
         raise ValueError("up and gate must be bfloat16 of one shape")
     _require_cuda(up, gate)
-    up, gate = up.contiguous(), gate.contiguous()
+    return _swiglu(up.contiguous(), gate.contiguous())
+
+
+def _swiglu(up, gate):
+    """swiglu() of operands that need no check."""
     out = torch.empty_like(up)
-    _lib.check(lib.rmoe_swiglu(up.data_ptr(), gate.data_ptr(), up.numel(), out.data_ptr(),
-                               _lib.stream_handle(up.device)))
+    _lib.check(_lib.load().rmoe_swiglu(up.data_ptr(), gate.data_ptr(), up.numel(),
+                                       out.data_ptr(), _lib.stream_handle(up.device)))
     return out
 
 

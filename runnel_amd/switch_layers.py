@@ -197,7 +197,7 @@ def swiglu(x: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     """silu(gate) * x; two plain bf16 GPU tensors of one shape in one launch,
     with the bits of the torch form."""
     if native.rows_ready(x, gate) and x.shape == gate.shape and x.numel() <= native.SWIGLU_MAX:
-        return native.swiglu(x, gate)
+        return native._swiglu(x, gate)
     return torch.nn.functional.silu(gate) * x
 
 

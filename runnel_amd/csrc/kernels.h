@@ -199,7 +199,7 @@ hipError_t static_scratch(hipStream_t stream, void** out);
 // *out = *word, then *word = 0 (one tiny kernel on `s`).
 hipError_t launch_take_status(uint32_t* word, uint32_t* out, hipStream_t s);
 
-int prefill_tile_rows(int T, int K, int E, int H, int I, int bits);
+int prefill_tile_rows(int T, int K, int E, int H, int I, int bits, bool shared);
 int prefill_max_mtiles(int T, int K, int E, int bm);
 int prefill_sort_slices(int T, int K);
 hipError_t launch_prefill(const PrefillArgs& a, int bits, bool combine, hipStream_t s);

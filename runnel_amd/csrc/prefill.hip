@@ -1306,8 +1306,8 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillArgs 
 // 32-row tiles waste few MFMA rows and spread few rows per expert over many
 // workgroups; 128-row tiles share each dequantised weight fragment across
 // more rows, but their workgroups must fill the device.  R = rows per expert
-// on average, W = the 128-row gate/up tiles they make (an expert's last tile
-// half full).  Whole block in us, 32- against 128-row tiles, 8 bits | 4 bits,
+// on average, W = the 128-row gate/up tiles of the call (an expert's last tile
+// half full, the shared expert's all full).  Whole block in us, 32- against 128-row tiles, 8 bits | 4 bits,
 // weights cold, hidden x intermediate x experts:
 //   R 30 to 48 pays from two workgroups per CU on (W 512): 2048 x 512 x 256
 //     at R 24 268/269 | 202/202, at 36 333/300 | 266/246; 3584 x 512 x 64 (W
@@ -1316,16 +1316,18 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillArgs 
 //     tile's fixed part) and for 4 bits (less weight to share): 2560 x 256 x
 //     60 at R 48 134/137 | 119/134, at 80 184/167 | 163/165, at 128 259/215 |
 //     233/212; 512 x 512 x 64 at R 64 69/71 | 62/70, at 128 96/86 | 88/85;
-//     2048 x 128 x 32 at R 128 93/103 | 86/102, at 384 203/179 | 181/176
-// Over 20 sizes x 13 values of R x both widths, blocks and switch calls, none
+//     2048 x 128 x 32 at R 128 93/103 | 86/102, at 384 203/179 | 181/176; one
+//     slot per token (half the rows are the shared expert's) 4096 x 256 x 32 at
+//     R 96 294/260, 4 bits at R 128 321/298
+// Over 27 sizes x 13 values of R x both widths, blocks and switch calls, none
 // is over 5% slower than with one line at R 48 (calls without a shared expert
 // would take 128 rows from R 24 on: up to 1.25 times as fast there).
-int prefill_tile_rows(int T, int K, int E, int H, int I, int bits) {
+int prefill_tile_rows(int T, int K, int E, int H, int I, int bits, bool shared) {
   const float R = (float)T * K / E;
   if (R <= 30.0f) return 32;
-  const float W = E * fmaxf(1.0f, R / 128 + 0.5f) * (I / 128);
+  const float W = (E * fmaxf(1.0f, R / 128 + 0.5f) + (shared ? T / 128 : 0)) * (I / 128);
   if (R <= 48.0f) return W >= 512 ? kPrefillBM : 32;
-  const float line = (850.0f + 600.0f * 1024 / H) * (bits == 4 ? 1.3f : 1.0f);
+  const float line = (850.0f + 600.0f * 1024 / H) * (bits == 4 ? 1.35f : 1.0f);
   return W * sqrtf(R) >= line ? kPrefillBM : 32;
 }
 
@@ -1412,7 +1414,7 @@ bool buffer_offsets_fit(const PrefillArgs& a, int bits) {
 
 hipError_t launch_prefill(const PrefillArgs& args, int bits, bool combine, hipStream_t s) {
   PrefillArgs a = args;
-  a.bm = prefill_tile_rows(a.T, a.K, a.E, a.H, a.I, bits);
+  a.bm = prefill_tile_rows(a.T, a.K, a.E, a.H, a.I, bits, a.has_shared != 0);
   if (a.bm == kPrefillBM && !buffer_offsets_fit(a, bits)) return hipErrorInvalidValue;
   const int nw = prefill_sort_slices(a.T, a.K);
   // one slice: the place kernel counts its rows itself

@@ -260,10 +260,10 @@ def test_long_prefill_skewed_routing_4bit(torch_cuda):
 
 
 @pytest.mark.parametrize("bits,T", [(8, 800), (8, 808), (8, 1022), (8, 1023), (4, 1496),
-                                    (4, 1504), (4, 1233), (4, 1234)])
+                                    (4, 1504), (4, 1266), (4, 1267)])
 def test_tile_height_rule(torch_cuda, bits, T):
     """Calls of a few experts with hundreds of rows each, on both sides of
-    the line (1023 and 1234 tokens here) from which a call takes
+    the line (1023 and 1267 tokens here) from which a call takes
     128-row tiles."""
     L = M.make_layer(77 + bits, hidden=256, inter=512, experts=8, top_k=4, bits=bits,
                      shared=False)

@@ -49,7 +49,7 @@
 extern "C" {
 #endif
 
-#define RMOE_ABI_VERSION 5
+#define RMOE_ABI_VERSION 6
 
 #define RMOE_OK 0
 #define RMOE_EINVAL (-1) /* inconsistent or unsupported shape / argument */
@@ -131,7 +131,9 @@ int rmoe_abi_version(void);
  * aligned. */
 int rmoe_rms_norm(const uint16_t* x, const uint16_t* weight, int32_t tokens, int32_t hidden,
                   float eps, uint16_t* out, void* stream);
-/* out[t] = bf16(sum_j weights[t, j] y[t, j] + sigmoid(gate[t]) shared[t]) in
+
+/* (This call and rmoe_swiglu came with ABI version 6.)
+ * out[t] = bf16(sum_j weights[t, j] y[t, j] + sigmoid(gate[t]) shared[t]) in
  * fp32, the slots in order, then the shared expert's row; with a residual
  * bf16(residual[t] + that).  The tail of mlx-lm's block around a SwitchGLU
  * (bench/mlx_lm_adapter.py:49-94) for rows that are already computed.

@@ -23,7 +23,7 @@ RMOE_ENULL = -6
 RMOE_ETIMEOUT = -7
 RMOE_EPLACEMENT = -8
 
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 EXPORTED = (
     "rmoe_abi_version", "rmoe_last_error", "rmoe_status_string",
@@ -97,6 +97,9 @@ def load() -> ctypes.CDLL:
         QP = ctypes.POINTER(QWeight)
         lib.rmoe_abi_version.restype = ctypes.c_int
         lib.rmoe_abi_version.argtypes = []
+        # before the symbols, which an older library may lack
+        if lib.rmoe_abi_version() != ABI_VERSION:
+            raise RuntimeError("librmoe.so ABI version mismatch; rebuild it")
         lib.rmoe_last_error.restype = ctypes.c_char_p
         lib.rmoe_last_error.argtypes = []
         lib.rmoe_status_string.restype = ctypes.c_char_p
@@ -137,8 +140,6 @@ def load() -> ctypes.CDLL:
                             "rmoe_router_workspace_bytes", "rmoe_chain_table_bytes",
                             "rmoe_workspace_status_offset"):
                 getattr(lib, name).restype = ctypes.c_int
-        if lib.rmoe_abi_version() != ABI_VERSION:
-            raise RuntimeError("librmoe.so ABI version mismatch; rebuild it")
         _lib = lib
         return lib
 

@@ -619,3 +619,17 @@ def test_row_kernels_give_way_to_torch_transforms():
     torch.jit.trace(note, x, check_trace=False)
     assert seen == [False] * 7
     assert not native.rows_ready(x.bfloat16())  # a host tensor
+
+
+def test_an_older_library_is_named_by_its_version(tmp_path, monkeypatch):
+    """A library of another ABI version is refused with that message, also
+    where it lacks symbols of this one."""
+    import subprocess
+    src = tmp_path / "old.c"
+    src.write_text(f"int rmoe_abi_version(void) {{ return {_lib.ABI_VERSION - 1}; }}\n")
+    old = tmp_path / "librmoe.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(old), str(src)], check=True)
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", old)
+    with pytest.raises(RuntimeError, match="ABI version"):
+        _lib.load()

@@ -144,3 +144,34 @@ def test_dequantize_from_the_longest_split_on(torch_cuda, bits, both):
         ref = (q.float() * s.float()).double() + b.double()
         assert torch.equal(b16.cpu(), ref.float().bfloat16())
         assert f32 is None or torch.equal(f32.cpu(), ref.float())
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+def test_quantize_a_whole_bank(torch_cuda, bits):
+    """128 experts of 512 x 2048 (134 M values): every word, scale and bias
+    equals the format's fp32 rules (correctly rounded division, halves to
+    even), evaluated by torch on the CPU."""
+    torch = torch_cuda
+    from runnel_amd import native
+    n = 2 ** bits - 1
+    g = torch.Generator(device="cuda").manual_seed(bits)
+    w = torch.randn((128, 512, 2048), generator=g, device="cuda") * 0.02
+    wq, s, b = (t.cpu() for t in native.quantize(w, bits))
+    w = w.cpu()
+    for e in range(0, 128, 16):
+        v = w[e:e + 16].reshape(-1, 64)
+        hi, lo = v.amax(1), v.amin(1)
+        mask = lo.abs() > hi.abs()
+        scale = ((hi - lo) / n).clamp_min(1e-7)
+        scale = torch.where(mask, scale, -scale)
+        edge = torch.where(mask, lo, hi)
+        q0 = (edge / scale).round()
+        scale = torch.where(q0 != 0, edge / q0, scale).bfloat16()
+        bias = torch.where(q0 == 0, torch.zeros_like(edge), edge).bfloat16()
+        q = (v - bias.float()[:, None]).div_(scale.float()[:, None]).round_().clamp_(0, n)
+        q = q.to(torch.uint8)
+        if bits == 4:
+            q = q[:, 0::2] | q[:, 1::2] << 4
+        assert torch.equal(s[e:e + 16].reshape(-1).view(torch.int16), scale.view(torch.int16))
+        assert torch.equal(b[e:e + 16].reshape(-1).view(torch.int16), bias.view(torch.int16))
+        assert torch.equal(wq[e:e + 16].reshape(q.shape[0], -1).view(torch.uint8), q)

@@ -39,7 +39,10 @@ def _scaled_x(seed, T, H, scale=4.0):
     return M.f32_to_bf16((rng.standard_normal((T, H)) * scale).astype(np.float32))
 
 
-@pytest.mark.parametrize("T,H,eps", [(7, 2048, 1e-6), (3, 320, 1e-2), (130, 512, 0.0)])
+@pytest.mark.parametrize("T,H,eps", [(7, 2048, 1e-6), (3, 320, 1e-2), (130, 512, 0.0),
+                                     # four and eight pieces a lane, and loops beyond
+                                     (5, 2040, 1e-6), (9, 2056, 1e-6), (5, 4096, 1e-5),
+                                     (3, 4104, 1e-6), (2, 8192, 0.0)])
 def test_rms_norm_bit_exact(torch_cuda, T, H, eps):
     torch = torch_cuda
     from runnel_amd import native

@@ -275,3 +275,23 @@ def test_sorted_block_router_choice(torch_cuda, router_bits, T):
         got, r = M.bf16_to_f32(host_bf16(out)), M.bf16_to_f32(ref)
         assert cosine(got.reshape(-1), r.reshape(-1)) >= MIN_COS
         assert np.abs(got - r).max() <= MAX_ABS
+
+
+@pytest.mark.parametrize("router_bits,T", [(None, 1024), (None, 1025), (8, 1025), (8, 2047),
+                                           (8, 2048), (8, 2049), (8, 3001)])
+def test_selection_from_many_tokens_on(torch_cuda, router_bits, T):
+    """Four selection waves a token up to 1024 tokens (2048 with an 8-bit
+    gate), one beyond, on logits whose K is split over two workgroups:
+    routing of sampled tokens, the last ones among them, bit-exact."""
+    torch = torch_cuda
+    from runnel_amd import native
+    print(f"selection: gate bits {router_bits}, {T} tokens", flush=True)
+    L = M.make_layer(400 + T, hidden=512, inter=128, experts=128, top_k=4,
+                     router_bits=router_bits)
+    x = M.make_x(23 + T, T, 512)
+    _, idx, scores = native.moe_block(layer_to_dev(L), dev_bf16(x), return_routing=True)
+    torch.cuda.synchronize()
+    at = np.unique(np.r_[np.random.default_rng(T).choice(T, 120, replace=False), 0, T - 2, T - 1])
+    ref_idx, ref_scores, _ = M.route(x[at], L.router_w, 4)
+    assert np.array_equal(idx.cpu().numpy()[at], ref_idx)
+    assert np.abs(scores.cpu().numpy()[at] - ref_scores).max() <= 2.0 ** -8

@@ -147,6 +147,56 @@ def test_rows_sharing_experts(torch_cuda, bits, Mr, N, K, E):
     assert np.linalg.norm(err) <= 4 * 2.0 ** -24 * np.linalg.norm(ref)
 
 
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("shift", [1, 2, 4])
+def test_scales_at_any_address(torch_cuda, bits, shift):
+    """Scales and biases 2, 4 and 8 bytes past a 16-byte boundary: only the
+    last suit the kernel that many rows share; the products are the same to
+    fp32 accuracy (K roundings; see test_rows_sharing_experts)."""
+    torch = torch_cuda
+    from runnel_amd import native
+    rng = np.random.default_rng(bits)
+    Mr, N, K, E = 128, 520, 1024, 4
+    w = rng.standard_normal((E, N, K), dtype=np.float32) * np.float32(0.02)
+    words, s, b = M.quantize(w, bits)
+    xb = M.make_x(11, Mr, K)
+    rhs = torch.from_numpy(rng.integers(0, E, Mr).astype(np.int32)).cuda()
+
+    def moved(a):
+        t = torch.empty(a.size + 8, dtype=torch.bfloat16, device="cuda")
+        v = t[shift:shift + a.size].view(a.shape)
+        v.copy_(dev_bf16(a))
+        return v
+
+    def product(sc, bi):
+        return native.gather_qmm(dev_bf16(xb), dev_i32(words), sc, bi, bits, rhs_indices=rhs,
+                                 out_dtype=torch.float32).double()
+    ref, got = product(dev_bf16(s), dev_bf16(b)), product(moved(s), moved(b))
+    assert torch.equal(got, ref) == (shift == 4)
+    assert (got - ref).norm() <= 8 * 2.0 ** -24 * ref.norm()
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_non_finite_row_stays_alone(torch_cuda, bits, bad):
+    """A row of x that holds a NaN or an infinity gives no finite output and
+    leaves the rows that share its expert as they are."""
+    torch = torch_cuda
+    from runnel_amd import native
+    rng = np.random.default_rng(7)
+    w = rng.standard_normal((2, 512, 1024), dtype=np.float32) * np.float32(0.02)
+    words, s, b = M.quantize(w, bits)
+    x = dev_bf16(M.make_x(12, 128, 1024))
+    rhs = (torch.arange(128, device="cuda") % 2).to(torch.int32)
+    dev = (dev_i32(words), dev_bf16(s), dev_bf16(b))
+    ref = native.gather_qmm(x, *dev, bits, rhs_indices=rhs)
+    x[37, 500] = bad
+    got = native.gather_qmm(x, *dev, bits, rhs_indices=rhs)
+    assert not got[37].isfinite().any()
+    keep = torch.arange(128, device="cuda") != 37
+    assert torch.equal(got[keep], ref[keep])
+
+
 @pytest.mark.parametrize("Mr,N,K,index", [
     (131072 + 600, 2048, 4096, "both"),   # qmv_rows_kernel, 2^15 threads a row
     (131072 + 600, 2048, 4096, "rhs"),    # and x in order

@@ -50,6 +50,32 @@ def test_combine(torch_cuda, T, k, H, shared, residual):
     assert (np.abs(f(host_bf16(out)) - ref) <= tol * 1.01 + 1e-30).all()
 
 
+def test_combine_non_finite(torch_cuda):
+    """Infinities and NaN in a slot's row, the shared row, the gate and the
+    residual reach the values they belong to and no others, as in the torch
+    form (slots past the call's k, which the kernel's batch of eight reads
+    again, add nothing)."""
+    torch = torch_cuda
+    from runnel_amd import native
+    g = torch.Generator().manual_seed(5)
+    T, k, H = 6, 3, 64
+    y = torch.randn((T, k, H), generator=g).bfloat16()
+    sh, res = torch.randn((2, T, H), generator=g).bfloat16()
+    gate = torch.randn((T, 1), generator=g).bfloat16()
+    w = torch.rand((T, k), generator=g)
+    y[0, k - 1, 3], y[1, 0, 5], y[1, 1, 5] = float("inf"), float("inf"), -float("inf")
+    sh[2, 7], res[3, 9], gate[4], gate[5] = float("nan"), -float("inf"), float("nan"), -float("inf")
+    w[0, 1] = 0.0
+    y[0, 1, 11] = float("inf")  # weight 0: NaN
+    ref = (y.float() * w[..., None]).sum(1) + torch.sigmoid(gate.float()) * sh.float()
+    ref = (res.float() + ref.bfloat16().float()).bfloat16().float()
+    got = native.combine(*(t.cuda() for t in (y, w, sh, gate, res))).cpu().float()
+    assert torch.equal(got.isnan(), ref.isnan())
+    assert torch.equal(got.isinf(), ref.isinf())
+    fin = ref.isfinite()
+    assert ((got - ref)[fin].abs() <= 2.0 ** -6 * ref[fin].abs() + 2.0 ** -7).all()
+
+
 @pytest.mark.parametrize("n", [1, 7, 8, 2049, 5 * 512])
 def test_swiglu(torch_cuda, n):
     torch = torch_cuda
@@ -148,3 +174,30 @@ def test_block_tail_under_forward_mode(torch_cuda):
         out = forward_ad.unpack_dual(blk(x, residual=forward_ad.make_dual(r, t)))
         assert torch.equal(out.primal, plain)  # (zero weights: the residual itself)
         assert torch.equal(out.tangent, t)
+
+
+def test_block_tail_torch_form(torch_cuda):
+    """Before packing, a residual that is not contiguous, not 16-byte aligned
+    or in autograd takes the torch form: the same values, and a gradient of
+    ones."""
+    torch = torch_cuda
+    from runnel_amd import SparseMoeBlock, native
+    blk = SparseMoeBlock(64, 64, 4, 2, shared_expert_intermediate_size=64, device="cuda")
+    w = torch.randn((4, 64, 64), device="cuda") * 0.1
+    for p in (blk.switch_mlp.gate_proj, blk.switch_mlp.up_proj, blk.switch_mlp.down_proj):
+        q, s, b = native.quantize(w, 8)
+        p.weight.copy_(q), p.scales.copy_(s), p.biases.copy_(b)
+    x, r = torch.randn(2, 5, 64, device="cuda").bfloat16()
+    plain = blk(x, residual=r).float()
+    wide = torch.zeros((5, 72), device="cuda").bfloat16()
+    wide[:, :64] = r
+    odd = torch.zeros(5 * 64 + 8, device="cuda").bfloat16()
+    odd[1:321] = r.reshape(-1)
+    grad = r.clone().requires_grad_()
+    for res in (wide[:, :64], odd[1:321].view(5, 64), grad):
+        assert not native.rows_ready(res)
+        out = blk(x, residual=res)
+        # the fp32 sum in another order: a step of bf16 at each of two roundings
+        assert ((out.float() - plain).abs() <= 2.0 ** -7 * (plain.abs() + r.float().abs())).all()
+    out.sum().backward()
+    assert torch.equal(grad.grad, torch.ones_like(grad))

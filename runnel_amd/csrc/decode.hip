@@ -2057,11 +2057,12 @@ bool router_mfma_eligible(int E, int H) {
 //   8-bit gate: 48 tokens 127.7/123.6 | 52.9/46.8 | 77.3/66.0; 56: 129.2/126.2
 //     | 52.6/47.9 | 77.9/67.8; 64: 130.9/131.2 | 54.7/51.7 | 78.4/68.9; 112: ..
 //     | 57.5/57.1 | 82.6/72.6; 128: .. | 59.4/61.0 | 83.5/76.9; 192: .. | .. |
-//     88.2/82.6; 256: .. | .. | 95.0/92.4.  Rows past 2048 take the selection's
+//     88.2/82.6; 256: .. | .. | 95.0/92.4.  The crossings lie between 14000
+//     (hidden 1024 x 256) and 18000 (2048 x 64).  Rows past 2048 take the selection's
 //     wide re-check: 4096 x 256 experts at 64 124.5/111.7, at 96 128.0/123.3,
 //     at 112 128.1/125.8; 4096 x 64 at 256 129.9/124.5, at 384 140.6/142.5
 bool router_direct(int T, int E, int H, bool rq8) {
-  return T * E <= (!rq8 ? 7168 : H > 2048 ? 24576 : 14336);
+  return T * E <= (!rq8 ? 7168 : H > 2048 ? 24576 : 15872);
 }
 
 // 64 x 64 tiles (two workgroups of four waves per CU) from 4096 tokens on,

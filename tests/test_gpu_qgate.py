@@ -252,10 +252,10 @@ def test_prefill_router_widest_rows(torch_cuda):
 
 
 @pytest.mark.parametrize("router_bits,T", [(None, 16), (None, 24), (None, 25), (8, 16), (8, 95),
-                                           (8, 96), (8, 97), (None, 112), (None, 113), (8, 224),
-                                           (8, 225)])
+                                           (8, 96), (8, 97), (None, 112), (None, 113), (8, 248),
+                                           (8, 249)])
 def test_sorted_block_router_choice(torch_cuda, router_bits, T):
-    """Either side of the token counts (here 112 and 224) where the
+    """Either side of the token counts (here 112 and 248) where the
     expert-sorted block changes from the one-launch router to the matrix-core
     one: routing bit-exact, scores within one bf16 step (their contract) on
     both."""

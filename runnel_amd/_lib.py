@@ -159,5 +159,11 @@ def ptr(t) -> int | None:
 
 
 def stream_handle(device=None) -> int:
+    """The current stream's hipStream_t on `device` (None: the current GPU),
+    without the Stream object that torch.cuda.current_stream makes."""
     import torch
-    return torch.cuda.current_stream(device).cuda_stream
+    if device is not None and not isinstance(device, torch.device):
+        device = torch.device(device)
+    index = None if device is None else device.index
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if index is None else index)

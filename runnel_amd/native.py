@@ -565,15 +565,21 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.
     return out.reshape(x.shape)
 
 
+_functorch_stack = torch._C._functorch.peek_interpreter_stack
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+_tracing_state = torch._C._get_tracing_state
+_is_compiling = torch.compiler.is_compiling
+
+
 def _plain_call() -> bool:
     """Whether nothing else has to see an operation's torch form: no
     forward-mode level, function transform (vmap, jvp, ...), dispatch or
     function mode (a default device aside), trace or compilation is active."""
-    if (forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch._C._len_torch_dispatch_stack() or torch.compiler.is_compiling()
-            or torch._C._get_tracing_state() is not None):
+    if (forward_ad._current_level >= 0 or _functorch_stack() is not None or _dispatch_modes()
+            or _tracing_state() is not None or _is_compiling()):
         return False
-    n = torch._C._len_torch_function_stack()
+    n = _function_modes()
     return n == 0 or all(isinstance(torch._C._get_function_stack_at(i), DeviceContext)
                          for i in range(n))
 
@@ -583,16 +589,14 @@ def rows_ready(*tensors) -> bool:
     every tensor a plain, contiguous, 16-byte aligned bf16 tensor of the
     current GPU outside autograd, and nothing that traces, transforms or
     intercepts torch operations active."""
-    for t in tensors:
-        if type(t) is not torch.Tensor or not t.is_cuda or t.dtype != BF16 or t.requires_grad:
-            return False
     if not _plain_call():
         return False
-    device = torch.cuda.current_device()
     for t in tensors:
-        if t.get_device() != device or not t.is_contiguous() or t.data_ptr() % 16:
+        if (type(t) is not torch.Tensor or not t.is_cuda or t.dtype != BF16 or t.requires_grad
+                or not t.is_contiguous() or t.data_ptr() % 16
+                or t.get_device() != tensors[0].get_device()):
             return False
-    return True
+    return tensors[0].get_device() == torch.cuda.current_device()
 
 
 def combine(y: torch.Tensor, weights: torch.Tensor, shared: torch.Tensor | None = None,

@@ -201,3 +201,12 @@ def test_block_tail_torch_form(torch_cuda):
         assert ((out.float() - plain).abs() <= 2.0 ** -7 * (plain.abs() + r.float().abs())).all()
     out.sum().backward()
     assert torch.equal(grad.grad, torch.ones_like(grad))
+
+
+def test_stream_handle_follows_the_current_stream(torch_cuda):
+    torch = torch_cuda
+    from runnel_amd import _lib
+    for stream in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(stream):
+            for device in (None, 0, "cuda", "cuda:0", torch.device("cuda"), torch.device("cuda:0")):
+                assert _lib.stream_handle(device) == stream.cuda_stream

@@ -630,9 +630,11 @@ struct Gemm {
     }
   }
   // Default cache policy: a load takes 64 bytes of each of 16 rows, half a
-  // line, and the other half is the next load's.  Non-temporal requests fetch
-  // the line again (read alone, 575 MB in this pattern: 5.29 TB/s against 5.72;
-  // 512 tokens 8-bit, gate/up 141 -> 126 us, down 70 -> 65).
+  // line, and the other half is the next load's, which then finds it in the
+  // L1.  Non-temporal loads asked L2 for each half: 12.2 M requests per 512
+  // token gate/up launch against 7.5 M, down 5.2 M against 3.0 (the bytes from
+  // memory went 649 -> 716 MB and 306 -> 292; gate/up 141 -> 126 us, down 70
+  // -> 65; read alone, 575 MB in this pattern: 5.29 TB/s and 5.72).
   __device__ __forceinline__ void load_b(int ch, uint4 (&w)[QPW][C::LPC]) const {
 #pragma unroll
     for (int qq = 0; qq < QPW; ++qq)

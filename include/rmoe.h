@@ -222,7 +222,10 @@ size_t rmoe_switch_combine_workspace_bytes(const rmoe_qweight* gate_up,
  * (mx.quantized_matmul at prefill sizes, the reference's qmm_4d_tile,
  * native/shaders/quantized_qmm.metal:68-151): that one runs on the matrix
  * cores with every dequantised weight rounded to bf16 and fp32
- * accumulation. */
+ * accumulation.  Calls of many rows share an expert's weights between rows;
+ * their fp32 sums run in another order than those of few, so a row's last
+ * bits may differ between calls of different row counts.  Within a call a
+ * row's value depends on that row alone, and equal calls give equal bits. */
 int rmoe_gather_qmm(const uint16_t* x, int32_t x_rows,
                     const int32_t* lhs_indices, const int32_t* rhs_indices,
                     int32_t rows, const rmoe_qweight* w, uint16_t* y_bf16,

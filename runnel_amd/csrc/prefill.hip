@@ -1321,7 +1321,7 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillArgs 
 //     2048 x 128 x 32 at R 128 93/103 | 86/102, at 384 203/179 | 181/176; one
 //     slot per token (half the rows are the shared expert's) 4096 x 256 x 32 at
 //     R 96 294/260, 4 bits at R 128 321/298
-// Over 27 sizes x 13 values of R x both widths, blocks and switch calls, none
+// Over 26 sizes x 13 values of R x both widths, blocks and switch calls, none
 // is over 5% slower than with one line at R 48 (calls without a shared expert
 // would take 128 rows from R 24 on: up to 1.25 times as fast there).
 int prefill_tile_rows(int T, int K, int E, int H, int I, int bits, bool shared) {

@@ -576,8 +576,8 @@ def _plain_call() -> bool:
     """Whether nothing else has to see an operation's torch form: no
     forward-mode level, function transform (vmap, jvp, ...), dispatch or
     function mode (a default device aside), trace or compilation is active."""
-    if (forward_ad._current_level >= 0 or _functorch_stack() is not None or _dispatch_modes()
-            or _tracing_state() is not None or _is_compiling()):
+    if (_is_compiling() or forward_ad._current_level >= 0 or _functorch_stack() is not None
+            or _dispatch_modes() or _tracing_state() is not None):
         return False
     n = _function_modes()
     return n == 0 or all(isinstance(torch._C._get_function_stack_at(i), DeviceContext)

@@ -633,3 +633,17 @@ def test_an_older_library_is_named_by_its_version(tmp_path, monkeypatch):
     monkeypatch.setattr(_lib, "LIB_PATH", old)
     with pytest.raises(RuntimeError, match="ABI version"):
         _lib.load()
+
+
+def test_swiglu_traces_as_its_torch_form():
+    """Compiled without graph breaks, traced to a graph and batched, the
+    SwiGLU is silu and a product, as the check for its kernel gives way."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from runnel_amd.switch_layers import swiglu
+    x, g = torch.randn(2, 4, 8).bfloat16()
+    ref = torch.nn.functional.silu(g) * x
+    assert torch.equal(torch.compile(swiglu, fullgraph=True, backend="eager")(x, g), ref)
+    ops = [n.target for n in make_fx(swiglu)(x, g).graph.nodes if n.op == "call_function"]
+    assert ops == [torch.ops.aten.silu.default, torch.ops.aten.mul.Tensor]
+    assert torch.equal(torch.vmap(swiglu)(x, g), ref)
